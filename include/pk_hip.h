@@ -427,8 +427,8 @@ int pk_hip_force_tiling(int index);
 int pk_hip_force_split(int splits);
 
 /* Tests and tuning: 0 makes every later search load its LSTM, jpred and
- * jout panels from memory each token even where they fit resident (gate
- * panels in registers, the joint's panels in LDS, loaded once a launch:
+ * jout panels from memory each token even where they fit resident (in its
+ * workgroups' registers, loaded once a launch:
  * P and J up to 640, at most 2 LSTM layers), 1 restores that; returns the
  * previous setting. Both compute the same tokens. */
 int pk_hip_force_search_resident(int on);

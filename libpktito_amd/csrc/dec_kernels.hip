@@ -97,18 +97,6 @@ __device__ __forceinline__ int panel_sum(const v4i (&wv)[KU], uint32_t kr, const
     return s;
 }
 
-/* panel_sum over a panel kept in LDS: unit u's bytes at wl + 1 KB u, in
- * the order panel_load reads them (lane l's 16 bytes at 16 l) */
-template <int KU>
-__device__ __forceinline__ int panel_sum_lds(const int8_t *wl, uint32_t kr, const int8_t *q, int lane) {
-    v4i wv[KU];
-#pragma unroll
-    for (int u = 0; u < KU; u++)
-        if (u < (int)kr)
-            wv[u] = *(const v4i *)(wl + u * kUnitBytes + lane * 16);
-    return panel_sum<KU>(wv, kr, q, lane);
-}
-
 /* Whether a kernel of KU units a panel loads its panels behind its row,
  * before the quantize (one memory round trip instead of two): where the
  * panels fit the registers beside the row (the 64-unit kernels load them
@@ -378,57 +366,15 @@ __device__ __forceinline__ float4 crow4(const float *x, uint32_t i, uint32_t n) 
                        k + 2 < n ? cload(x + k + 2) : 0.0f, k + 3 < n ? cload(x + k + 3) : 0.0f);
 }
 
-template <int CH, int KU, bool RES>
+template <int CH, int KU>
 __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
     __shared__ __attribute__((aligned(16))) int8_t q0[64 * KU], q1[64 * KU];
     __shared__ float dq[2], gates[4][16];
     __shared__ uint32_t shared_u[3];
-    /* RES: the jpred panel wg (slot 0) and the jout panels wg and wg + G
-     * (slots 1, 2) of this workgroup, loaded once */
-    __shared__ __attribute__((aligned(16))) int8_t wres[RES ? 3 : 1][RES ? KU * kUnitBytes : 16];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint32_t G = gridDim.x, wg = blockIdx.x;
     const uint32_t P = a.P, J = a.J;
     uint32_t nbar = 0;
-
-    /* RES: each wave's gate panels of every LSTM layer (wx and wh, kResLayers
-     * at most) held in registers for the whole segment, with their rows'
-     * scales and biases; waves 1-3 the scale and bias of their jpred / jout
-     * row */
-    constexpr int RL = RES ? kResLayers : 1, RU = RES ? KU : 1;
-    v4i rwx[RL][RU], rwh[RL][RU];
-    float rxs[RL], rhs[RL], rb[RL], jsr = 0.0f, jbr = 0.0f;
-    if constexpr (RES) {
-        if (wg < P / 16) {
-            const uint32_t j0 = 16 * wg, pn = (wv * P + j0) / 16, r = wv * P + j0 + (lane & 15);
-#pragma unroll
-            for (int l = 0; l < RL; l++)
-                if (l < (int)a.L) {
-                    panel_load<KU>(a.wx[l], a.lstm_stride, pn, a.kr_p, lane, rwx[l]);
-                    panel_load<KU>(a.wh[l], a.lstm_stride, pn, a.kr_p, lane, rwh[l]);
-                    rxs[l] = a.wxs[l][r];
-                    rhs[l] = a.whs[l][r];
-                    rb[l] = a.b[l] ? a.b[l][r] : 0.0f;
-                }
-        }
-        if (wv >= 1) {
-            const bool jp = wv == 1;
-            const uint32_t pn = jp ? wg : wg + (wv - 2) * G, panels = jp ? J / 16 : a.rows_out / 16;
-            if (pn < panels) {
-                const uint32_t kr = jp ? a.kr_p : a.kr_j, r = 16 * pn + (lane & 15);
-                v4i t[KU];
-                panel_load<KU>(jp ? a.jpred : a.jout, jp ? a.jpred_stride : a.jout_stride, pn, kr, lane, t);
-#pragma unroll
-                for (int u = 0; u < KU; u++)
-                    if (u < (int)kr)
-                        *(v4i *)(wres[wv - 1] + u * kUnitBytes + lane * 16) = t[u];
-                const float *bb = jp ? a.jpred_b : a.jout_b;
-                jsr = (jp ? a.jpred_s : a.jout_s)[r];
-                jbr = bb ? bb[r] : 0.0f;
-            }
-        }
-        __syncthreads();
-    }
 
     /* the grid barrier: this workgroup's stores have landed, then it counts
      * itself in and waits for the G arrivals of barrier nbar; false (leave)
@@ -480,16 +426,11 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
         else if (wv == 1)
             load_row<CH>([&](uint32_t i) { return crow4(h_in, i, P); }, P, lane, v);
         const uint32_t pn = (wv * P + j0) / 16;
-        v4i wxv[RES ? 1 : KU], whv[RES ? 1 : KU];
-        float wxsr = 0.0f, whsr = 0.0f, br = 0.0f;
-        if constexpr (!RES) {
-            panel_load<KU>(a.wx[l], a.lstm_stride, pn, a.kr_p, lane, wxv);
-            panel_load<KU>(a.wh[l], a.lstm_stride, pn, a.kr_p, lane, whv);
-            const uint32_t r = wv * P + j0 + (lane & 15);
-            wxsr = a.wxs[l][r];
-            whsr = a.whs[l][r];
-            br = a.b[l] ? a.b[l][r] : 0.0f;
-        }
+        v4i wxv[KU], whv[KU];
+        panel_load<KU>(a.wx[l], a.lstm_stride, pn, a.kr_p, lane, wxv);
+        panel_load<KU>(a.wh[l], a.lstm_stride, pn, a.kr_p, lane, whv);
+        const uint32_t r = wv * P + j0 + (lane & 15);
+        const float wxsr = a.wxs[l][r], whsr = a.whs[l][r], br = a.b[l] ? a.b[l][r] : 0.0f;
         const float cold = threadIdx.x < 16 ? cload(c + j0 + threadIdx.x) : 0.0f;
         if (wv == 0) {
             const float d = quant_loaded<CH>(v, P, a.kr_p, q0, lane);
@@ -501,21 +442,7 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
                 dq[1] = d;
         }
         __syncthreads();
-        int sx = 0, sh = 0;
-        if constexpr (RES) {
-#pragma unroll
-            for (int k = 0; k < RL; k++)
-                if (k == (int)l) {
-                    sx = panel_sum<KU>(rwx[k], a.kr_p, q0, lane);
-                    sh = panel_sum<KU>(rwh[k], a.kr_p, q1, lane);
-                    wxsr = rxs[k];
-                    whsr = rhs[k];
-                    br = rb[k];
-                }
-        } else {
-            sx = panel_sum<KU>(wxv, a.kr_p, q0, lane);
-            sh = panel_sum<KU>(whv, a.kr_p, q1, lane);
-        }
+        const int sx = panel_sum<KU>(wxv, a.kr_p, q0, lane), sh = panel_sum<KU>(whv, a.kr_p, q1, lane);
         if (lane < 16) {
             const float g = gemv_out(sx, dq[0], wxsr, a.b[l], br);
             gates[wv][lane] = g + gemv_out(sh, dq[1], whsr, nullptr, 0.0f);
@@ -561,28 +488,6 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
         }
     };
 
-    /* RES: the row quantized by wave 0, then wave w1 sums the panel pn
-     * kept in LDS slot w1 - 1 (jpred: wave 1, panel wg; jout: waves 2 and
-     * 3, panels wg and wg + G) */
-    auto gemv_res = [&](auto value4, uint32_t n, uint32_t kr, const float *bias, uint32_t panels, float *out,
-                        bool joint) {
-        float4 v[CH];
-        if (wv == 0) {
-            load_row<CH>(value4, n, lane, v);
-            const float d = quant_loaded<CH>(v, n, kr, q0, lane);
-            if (lane == 0)
-                dq[0] = d;
-        }
-        __syncthreads();
-        const bool mine = joint ? wv >= 2 : wv == 1;
-        const uint32_t pn = joint ? wg + (wv - 2) * G : wg;
-        if (mine && pn < panels) {
-            const int s = panel_sum_lds<KU>(wres[wv - 1], kr, q0, lane);
-            if (lane < 16)
-                cstore(out + 16 * pn + lane, gemv_out(s, dq[0], jsr, bias, jbr));
-        }
-    };
-
     uint32_t cur = 0;                               /* bit l: which of layer l's two h buffers is current */
     auto predict = [&](uint32_t label) -> bool {
         const float *x = a.embed + (size_t)label * P;
@@ -597,11 +502,8 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
             x = h_out;
         }
         const float *hl = x;
-        if constexpr (RES)
-            gemv_res([&](uint32_t i) { return crow4(hl, i, P); }, P, a.kr_p, a.jpred_b, J / 16, a.gp, false);
-        else
-            gemv([&](uint32_t i) { return crow4(hl, i, P); }, P, a.kr_p, a.jpred, a.jpred_stride, a.jpred_s,
-                 a.jpred_b, J / 16, a.gp);
+        gemv([&](uint32_t i) { return crow4(hl, i, P); }, P, a.kr_p, a.jpred, a.jpred_stride, a.jpred_s, a.jpred_b,
+             J / 16, a.gp);
         return barrier();
     };
 
@@ -614,10 +516,7 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
             return make_float4(relu_sum(fv.x, gv.x), relu_sum(fv.y, gv.y), relu_sum(fv.z, gv.z),
                                relu_sum(fv.w, gv.w));
         };
-        if constexpr (RES)
-            gemv_res(zrow, J, a.kr_j, a.jout_b, a.rows_out / 16, a.logit, true);
-        else
-            gemv(zrow, J, a.kr_j, a.jout, a.jout_stride, a.jout_s, a.jout_b, a.rows_out / 16, a.logit);
+        gemv(zrow, J, a.kr_j, a.jout, a.jout_stride, a.jout_s, a.jout_b, a.rows_out / 16, a.logit);
         if (!barrier())
             return false;
         if (wv == 0) {
@@ -669,6 +568,408 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
             return;
         if (lasts >= a.max_symbols && last == t)
             t++;
+    }
+    if (wg == 0 && threadIdx.x == 0) {
+        a.out[0] = ntoks;
+        a.out[1] = status;
+    }
+}
+
+/* The resident search: the same search where every panel fits the chip's
+ * registers (a.L <= kResLayers, panels of kResUnits units), each workgroup of
+ * eight waves holding its rows of every matrix for the whole segment: waves
+ * 0 to 3 a gate each of 16 units' wx rows of every layer, waves 4 to 7 their
+ * wh rows; wave 4 a jpred panel too, waves 5 and 6 a jout panel each. What
+ * bounds it is the exchange between workgroups, four of them a token (each
+ * layer's h, gp, the joint's best), so an exchange is one trip through
+ * memory: every value travels as one 64-bit word with the number of the step
+ * it belongs to (agent scope, coherent across the XCDs' L2s), and its readers
+ * poll the values themselves. A barrier and a load after it, as the streaming
+ * kernel above has them, are three trips.
+ *
+ * Words are never overwritten while someone may still read them: each h and
+ * gp word changes once a prediction, and between two predictions lies a
+ * joint, whose words every workgroup writes (its two panels' bests, empty
+ * where it has none) only after it has read h and gp, and reads whole before
+ * it goes on; the joint's own words alternate between two sets. Words start
+ * at zero and steps count from 1.
+ *
+ * The joint's logits do not travel: a panel's wave reduces its 16 to the
+ * best (argmax_wave's rule: a key ordered as the values are, both zeros
+ * alike, NaN below all, a NaN at token 0 above all; the first of equal keys),
+ * the durations' travel as keys. Between two exchanges wave 0 polls and
+ * quantizes and nothing else: the wh half of a layer's step needs only the h
+ * that the prediction before made, so waves 4 to 7 sum it while the h moves
+ * on, and wave 7 keeps frames in a ring in LDS up to kRingFrames ahead.
+ * Waits are bounded as above.
+ *
+ * Measured, the model's shapes (40 workgroups), 384 frames with 123 tokens
+ * and 133 joints: 1.29 ms a launch where the same panels resident with a
+ * barrier an exchange took 2.89 ms; of an exchange's 2.6 us, 1.55 us is the
+ * wait for the words, 0.35 us the row's quantize, 0.45 us the sums and the
+ * activations (with v_dot4 chains and one lane a whole cell: 1.4 us). */
+constexpr int kRingFrames = 8;
+
+/* (non-NaN) values as unsigned keys in the order of the values, +0 and -0
+ * one key, above 0; NaN: 0 */
+__device__ __forceinline__ uint32_t order_key(float v) {
+    const uint32_t b = __float_as_uint(v + 0.0f);
+    return v == v ? ((b & 0x80000000u) ? ~b : b | 0x80000000u) : 0u;
+}
+
+/* the largest of the wave's, all lanes active (wave_max_nonneg's steps) */
+__device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+/* chunk i of a row of whole chunks, from any float's address (one 16-byte
+ * load: the hardware takes it at 4-byte alignment) */
+typedef float v4fu __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 row4u(const float *x, uint32_t i) {
+    const v4fu v = *(const v4fu *)(x + 4 * i);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+/* The resident panels have KU units always, those past the matrix zero, so
+ * their sums have no branches (whatever bytes q holds there meet zeros). */
+template <int KU>
+__device__ __forceinline__ void panel_load_whole(const int8_t *__restrict__ w, uint64_t wstride, uint32_t p,
+                                                 uint32_t kr, int lane, v4i (&wv)[KU]) {
+    const int8_t *wp = w + (size_t)p * kUnitBytes + lane * 16;
+#pragma unroll
+    for (int u = 0; u < KU; u++)
+        wv[u] = u < (int)kr ? *(const v4i *)(wp + (size_t)u * wstride) : v4i{ 0, 0, 0, 0 };
+}
+
+/* The sums of a panel's 16 rows on the matrix cores: the unit's 16 rows by
+ * 64 inputs are an operand as they are, the vector is the other one's every
+ * column (lane l holds inputs 16 (l / 16) .. + 15, whatever its column), so
+ * lane l gets rows 4 (l / 16) + 0 .. 3 with no exchange between lanes, and
+ * keeps row_of(l). Exact int32 sums, two chains. */
+__device__ __forceinline__ int row_of(int lane) { return 4 * (lane >> 4) + (lane & 3); }
+
+template <int KU>
+__device__ __forceinline__ int panel_sum_whole(const v4i (&wv)[KU], const int8_t *q, int lane) {
+    const int8_t *qp = q + (lane >> 4) * 16;
+    v4i s[2] = { { 0, 0, 0, 0 }, { 0, 0, 0, 0 } };
+#pragma unroll
+    for (int u = 0; u < KU; u++)
+        s[u & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[u], *(const v4i *)(qp + 64 * u), s[u & 1], 0, 0, 0);
+    s[0] += s[1];
+    const int lo = lane & 1 ? s[0][1] : s[0][0], hi = lane & 1 ? s[0][3] : s[0][2];
+    return lane & 2 ? hi : lo;
+}
+
+__device__ __forceinline__ uint64_t wload(const uint64_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void wstore(uint64_t *p, uint32_t hi, uint32_t lo) {
+    __hip_atomic_store(p, (uint64_t)hi << 32 | lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(512) void search_resident_kernel(SearchArgs a) {
+    constexpr int KU = kResUnits, RL = kResLayers, CH = (16 * KU + 63) / 64;
+    __shared__ __attribute__((aligned(16))) int8_t qx[64 * KU], qh[RL][64 * KU];
+    __shared__ float dx, dh[RL], gates[4][16], hsum[RL][4][16];
+    __shared__ uint32_t s_tok, s_dur, s_bad;
+    __shared__ __attribute__((aligned(16))) float ring[kRingFrames][64 * KU];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t G = gridDim.x, wg = blockIdx.x, P = a.P, J = a.J, T = a.T;
+    const bool has_units = wg < P / 16;
+    const int row = row_of(lane);                   /* this lane's row of a panel; */
+    const bool own = (lane & 12) == 0;              /* four lanes have it, the first speaks for it */
+
+    /* everything this workgroup keeps, loaded once: wr the wave's gate panel
+     * of each layer's wx or wh with its rows' scales and wx's biases, wj its
+     * jpred or jout panel */
+    v4i wr[RL][KU], wj[KU];
+    float rs[RL], rb[RL], creg[RL], jsr = 0.0f, jbr = 0.0f;
+#pragma unroll
+    for (int l = 0; l < RL; l++) {
+        rs[l] = rb[l] = creg[l] = 0.0f;
+        if (has_units && l < (int)a.L) {
+            const uint32_t pn = ((wv & 3) * P) / 16 + wg, r = 16 * pn + row;
+            panel_load_whole<KU>(wv < 4 ? a.wx[l] : a.wh[l], a.lstm_stride, pn, a.kr_p, lane, wr[l]);
+            rs[l] = (wv < 4 ? a.wxs[l] : a.whs[l])[r];
+            rb[l] = wv < 4 && a.b[l] ? a.b[l][r] : 0.0f;
+        }
+    }
+    const bool jp = wv == 4, jo = wv == 5 || wv == 6;
+    const uint32_t my_panel = jp ? wg : wg + (wv - 5) * G;
+    const bool mine = (jp && my_panel < J / 16) || (jo && my_panel < a.rows_out / 16);
+    if (mine) {
+        const uint32_t r = 16 * my_panel + row;
+        panel_load_whole<KU>(jp ? a.jpred : a.jout, jp ? a.jpred_stride : a.jout_stride, my_panel,
+                             jp ? a.kr_p : a.kr_j, lane, wj);
+        const float *bb = jp ? a.jpred_b : a.jout_b;
+        jsr = (jp ? a.jpred_s : a.jout_s)[r];
+        jbr = bb ? bb[r] : 0.0f;
+    }
+    if (threadIdx.x == 0)
+        s_bad = 0;
+
+    /* wave 0: load() until it finds every word it wants (a lane's ok); s_bad
+     * past the iteration limit or where another workgroup has given up */
+    auto poll = [&](auto load) {
+        for (uint32_t it = 0;;) {
+            if (__ballot(load()) == __builtin_amdgcn_read_exec())
+                return;
+            if (++it >= a.spin || ((it & 63) == 0 && __hip_atomic_load(a.sync + 1, __ATOMIC_RELAXED,
+                                                                       __HIP_MEMORY_SCOPE_AGENT))) {
+                if (lane == 0) {
+                    __hip_atomic_store(a.sync + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    s_bad = 1;
+                }
+                return;
+            }
+        }
+    };
+    /* wave 0: n words (a multiple of 16, at most 64 KU) of step tag into v,
+     * a lane's chunks as load_row has them */
+    auto poll_row = [&](const uint64_t *w, uint32_t n, uint32_t tag, float4 (&v)[CH]) {
+        poll([&]() {
+            uint64_t x[CH][4];
+#pragma unroll
+            for (int c = 0; c < CH; c++) {
+                const uint32_t i = lane + 64 * c;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    x[c][e] = 4 * i < n ? wload(w + 4 * i + e) : (uint64_t)tag;
+            }
+            bool ok = true;
+#pragma unroll
+            for (int c = 0; c < CH; c++) {
+                v[c] = make_float4(__uint_as_float((uint32_t)(x[c][0] >> 32)), __uint_as_float((uint32_t)(x[c][1] >> 32)),
+                                   __uint_as_float((uint32_t)(x[c][2] >> 32)), __uint_as_float((uint32_t)(x[c][3] >> 32)));
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    ok = ok && (uint32_t)x[c][e] == tag;
+            }
+            return ok;
+        });
+    };
+
+    /* the ring holds frames max(lo, hi - kRingFrames) .. hi - 1; wave 7 adds
+     * the next four at most of frames from .. from + kRingFrames - 1 (a zero
+     * duration comes back to frame from, which stays) */
+    uint32_t lo = 0, hi = 0;
+    auto ring_fill = [&](uint32_t from) {
+        if (from > hi)
+            lo = hi = from;
+        const uint32_t end = min(min(from + (uint32_t)kRingFrames, T), hi + 4);
+        if (wv == 7) {
+            float4 v[4][CH];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (hi + k < end) {
+                    const float *fr = a.f + (size_t)(hi + k) * J;
+                    load_row<CH>([&](uint32_t i) { return row4u(fr, i); }, J, lane, v[k]);
+                }
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (hi + k < end)
+#pragma unroll
+                    for (int c = 0; c < CH; c++)
+                        if (4 * (lane + 64 * c) < J)
+                            *(float4 *)&ring[(hi + k) % kRingFrames][4 * (lane + 64 * c)] = v[k][c];
+        }
+        hi = hi > end ? hi : end;
+    };
+    ring_fill(0);
+    /* the first prediction's h is zero: a row quantized to d = 0 and sums 0 */
+    if (wv >= 4 && own)
+#pragma unroll
+        for (int l = 0; l < RL; l++)
+            hsum[l][wv - 4][row] = gemv_out(0, 0.0f, rs[l], nullptr, 0.0f);
+    __syncthreads();
+
+    uint32_t step = 0, jstep = 0;                   /* predictions and joints so far */
+    bool fresh = false;                             /* gp not read since the last prediction */
+    float4 vg[CH];
+
+    /* layer l's step of units 16 wg .. + 15 from the quantized x and the wh
+     * half at hand: wave w's gate with its activation, then, the gates met in
+     * LDS, the cell and the word of each unit's h; l is a constant at every
+     * call */
+    auto gate = [&](int l, const int8_t *q, float d) {
+        float g = gemv_out(panel_sum_whole<KU>(wr[l], q, lane), d, rs[l], a.b[l], rb[l]);
+        g = g + hsum[l][wv][row];
+        g = wv == 2 ? pk_tanhf(g) : pk_sigmoidf(g);
+        if (own)
+            gates[wv][row] = g;
+    };
+    auto cell = [&](int l) {
+        if (threadIdx.x < 16) {
+            const uint32_t t = threadIdx.x;
+            const float cj = gates[1][t] * creg[l] + gates[0][t] * gates[2][t];
+            creg[l] = cj;
+            wstore(a.hw + (size_t)l * P + 16 * wg + t, __float_as_uint(gates[3][t] * pk_tanhf(cj)), step);
+        }
+    };
+
+    auto predict = [&](uint32_t label) -> bool {
+        step++;
+        fresh = true;
+        if (wv == 0 && has_units) {
+            float4 v[CH];
+            const float *x = a.embed + (size_t)label * P;
+            load_row<CH>([&](uint32_t i) { return row4u(x, i); }, P, lane, v);
+            const float d = quant_loaded<CH>(v, P, a.kr_p, qx, lane);
+            if (lane == 0)
+                dx = d;
+        }
+        __syncthreads();
+        if (has_units && wv < 4)
+            gate(0, qx, dx);
+        __syncthreads();
+#pragma unroll
+        for (int l = 0; l < RL; l++)
+            if (l < (int)a.L) {
+                /* h of layer l whole: the next layer's x (or jpred's row) and
+                 * this layer's h_in of the next prediction */
+                const bool last = l + 1 == (int)a.L;
+                if (wv == 0) {
+                    if (has_units)
+                        cell(l);
+                    float4 v[CH];
+                    poll_row(a.hw + (size_t)l * P, P, step, v);
+                    const float d = quant_loaded<CH>(v, P, a.kr_p, qh[l], lane);
+                    if (lane == 0)
+                        dh[l] = d;
+                }
+                __syncthreads();
+                if (s_bad)
+                    return false;
+                if (last && jp && mine) {
+                    const float o = gemv_out(panel_sum_whole<KU>(wj, qh[l], lane), dh[l], jsr, a.jpred_b, jbr);
+                    if (own)
+                        wstore(a.gpw + 16 * my_panel + row, __float_as_uint(o), step);
+                }
+                if (has_units) {
+                    if (wv >= 4) {
+                        const float o = gemv_out(panel_sum_whole<KU>(wr[l], qh[l], lane), dh[l], rs[l], nullptr, 0.0f);
+                        if (own)
+                            hsum[l][wv - 4][row] = o;
+                    } else if (!last && l + 1 < RL) {
+                        gate(l + 1 < RL ? l + 1 : l, qh[l], dh[l]);
+                    }
+                }
+                if (!last)
+                    __syncthreads();
+            }
+        return true;
+    };
+
+    /* the joint at frame t: every panel's best out, all of them in */
+    auto joint = [&](uint32_t t, uint32_t &k, uint32_t &di) -> bool {
+        jstep++;
+        const uint32_t tag = jstep & 0xfffffu;
+        uint64_t *tw = a.jw + (size_t)(jstep & 1) * kJointWords, *dw = tw + 128;
+        if (wv == 0) {
+            float4 v[CH];
+            if (t >= lo && t < hi && hi - t <= (uint32_t)kRingFrames)
+                load_row<CH>([&](uint32_t i) { return *(const float4 *)&ring[t % kRingFrames][4 * i]; }, J, lane, v);
+            else
+                load_row<CH>([&](uint32_t i) { return row4u(a.f + (size_t)t * J, i); }, J, lane, v);
+            if (fresh)
+                poll_row(a.gpw, J, step, vg);
+#pragma unroll
+            for (int c = 0; c < CH; c++)
+                v[c] = 4 * (lane + 64 * c) < J
+                           ? make_float4(relu_sum(v[c].x, vg[c].x), relu_sum(v[c].y, vg[c].y),
+                                         relu_sum(v[c].z, vg[c].z), relu_sum(v[c].w, vg[c].w))
+                           : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const float d = quant_loaded<CH>(v, J, a.kr_j, qx, lane);
+            if (lane == 0)
+                dx = d;
+        }
+        fresh = false;
+        __syncthreads();
+        if (s_bad)
+            return false;
+        if (jo) {
+            uint32_t best = 0, at = 0;
+            if (mine) {
+                const float v = gemv_out(panel_sum_whole<KU>(wj, qx, lane), dx, jsr, a.jout_b, jbr);
+                const uint32_t r = 16 * my_panel + row;
+                const uint32_t key = (r == 0 || r == a.V + 1) && v != v ? ~0u : order_key(v);
+                const uint32_t tk = r <= a.V ? key : 0u;
+                best = wave_max_u(tk);
+                at = 16 * my_panel + (uint32_t)row_of(__builtin_ctzll(__ballot(tk == best)));
+                if (own && r > a.V && r <= a.V + a.n_dur)
+                    wstore(dw + (r - a.V - 1), key, tag);
+            }
+            if (lane == 0)
+                wstore(tw + wg + (wv - 5) * G, best, (best ? at : 0u) << 20 | tag);
+        }
+        ring_fill(t);
+        if (wv == 0) {
+            uint64_t xa, xb, xd;
+            poll([&]() {
+                xa = lane < (int)(2 * G) ? wload(tw + lane) : (uint64_t)tag;
+                xb = 64 + lane < (int)(2 * G) ? wload(tw + 64 + lane) : (uint64_t)tag;
+                xd = lane < (int)a.n_dur ? wload(dw + lane) : (uint64_t)tag;
+                return ((uint32_t)xa & 0xfffffu) == tag && ((uint32_t)xb & 0xfffffu) == tag && (uint32_t)xd == tag;
+            });
+            const uint32_t ka = (uint32_t)(xa >> 32), kb = (uint32_t)(xb >> 32), kd = (uint32_t)(xd >> 32);
+            const uint32_t ma = wave_max_u(ka), mb = wave_max_u(kb), md = wave_max_u(kd);
+            const int la = __builtin_ctzll(__ballot(ka == ma)), lb = __builtin_ctzll(__ballot(kb == mb));
+            const uint32_t ta = (uint32_t)__builtin_amdgcn_readlane((int)((uint32_t)xa >> 20), la);
+            const uint32_t tb = (uint32_t)__builtin_amdgcn_readlane((int)((uint32_t)xb >> 20), lb);
+            const uint32_t ld = (uint32_t)__builtin_ctzll(__ballot(kd == md));
+            if (lane == 0) {
+                s_tok = mb > ma ? tb : ta;
+                s_dur = ld;
+            }
+        }
+        __syncthreads();
+        if (s_bad)
+            return false;
+        k = s_tok;
+        di = s_dur;
+        return true;
+    };
+
+    /* one copy of each phase's code: the first prediction is the blank's */
+    const uint32_t blank = a.blank;
+    uint32_t ntoks = 0, status = 0, k = blank, t = 0, last = 0xffffffffu, lasts = 0;
+    while (true) {
+        if (!predict(k))
+            return;
+        if (lasts >= a.max_symbols && last == t)
+            t++;
+        if (t >= T)
+            break;
+        uint32_t di, d, at;
+        do {
+            at = t;
+            if (!joint(t, k, di))
+                return;
+            d = (uint32_t)a.dur[di];
+            if (k == blank && d == 0)
+                d = 1;
+            t += d;
+        } while (k == blank && t < T);
+        if (k == blank)
+            break;
+        if (ntoks == a.cap) {
+            status = 2;
+            break;
+        }
+        if (wg == 0 && threadIdx.x == 0) {
+            a.toks[3 * ntoks] = (int32_t)k;
+            a.toks[3 * ntoks + 1] = (int32_t)at;
+            a.toks[3 * ntoks + 2] = a.dur[di];
+        }
+        ntoks++;
+        lasts = last == at ? lasts + 1 : 1;
+        last = at;
     }
     if (wg == 0 && threadIdx.x == 0) {
         a.out[0] = ntoks;
@@ -752,10 +1053,15 @@ bool set_search_resident(bool on) {
     return was;
 }
 
+/* The workspace: the flags, the tokens, then what the kernel's workgroups
+ * exchange: h, c, gp and the logits of the streaming kernel, or the resident
+ * kernel's words (h's and gp's, and the joint's two sets). */
+static size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
+
 size_t search_workspace_bytes(uint32_t L, uint32_t P, uint32_t J, uint32_t rows_out, uint32_t cap) {
-    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    return up(512) + up((size_t)L * 2 * P * 4) + up((size_t)L * P * 4) + up((size_t)J * 4) + up((size_t)rows_out * 4) +
-           up((size_t)cap * 12) + up(8);
+    const size_t loaded = up256((size_t)L * P * 4) + up256((size_t)J * 4) + up256((size_t)rows_out * 4);
+    const size_t words = up256((size_t)J * 8) + up256((size_t)2 * kJointWords * 8);
+    return up256(512) + up256((size_t)cap * 12) + up256((size_t)L * P * 8) + (loaded > words ? loaded : words) + 256;
 }
 
 int launch_search(SearchArgs &a, void *ws, hipStream_t s) {
@@ -763,31 +1069,10 @@ int launch_search(SearchArgs &a, void *ws, hipStream_t s) {
         a.L > (uint32_t)kMaxDecLayers || a.rows_out % 16 || a.V + 1 + a.n_dur > a.rows_out || a.n_dur == 0 ||
         a.n_dur > 64 || a.V + 1 > 64 * 32 || 64 * a.kr_p < a.P || a.kr_p > 16 || 64 * a.kr_j < a.J || a.kr_j > 16)
         return -2;
-    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    char *p = (char *)ws;
-    a.sync = (uint32_t *)p;
-    p += up(512);
-    a.h = (float *)p;
-    p += up((size_t)a.L * 2 * a.P * 4);
-    a.c = (float *)p;
-    p += up((size_t)a.L * a.P * 4);
-    a.gp = (float *)p;
-    p += up((size_t)a.J * 4);
-    a.logit = (float *)p;
-    p += up((size_t)a.rows_out * 4);
-    a.toks = (int32_t *)p;
-    p += up((size_t)a.cap * 12);
-    a.out = (uint32_t *)p;
-    /* the arrivals, the flag and the state start at zero (c and h: the
-     * reference zeroes them a segment, core/decoder.c:158-165); the logits,
-     * gp and the tokens are written before they are read */
-    if (hipMemsetAsync(a.sync, 0, 512, s) != hipSuccess ||
-        hipMemsetAsync(a.h, 0, up((size_t)a.L * 2 * a.P * 4) + up((size_t)a.L * a.P * 4), s) != hipSuccess ||
-        hipMemsetAsync(a.out, 0, 8, s) != hipSuccess)
-        return -1;
     /* resident: every panel's units and every layer's gate panels fit
      * (kr <= kResUnits, L <= kResLayers), one workgroup a jpred panel and
-     * two a jout panel's pair; else the panels are loaded each token */
+     * two a jout panel's pair (their words are read two a lane of one wave);
+     * else the panels are loaded each token */
     uint32_t Gr = a.P / 16;
     Gr = Gr > a.J / 16 ? Gr : a.J / 16;
     Gr = Gr > (a.rows_out / 16 + 1) / 2 ? Gr : (a.rows_out / 16 + 1) / 2;
@@ -800,9 +1085,37 @@ int launch_search(SearchArgs &a, void *ws, hipStream_t s) {
         G = Gr;
     if (G > 64)
         return -2;                              /* the barrier reads every workgroup's slot in one wave */
+    char *p = (char *)ws;
+    a.sync = (uint32_t *)p;
+    a.out = a.sync + 2;
+    p += up256(512);
+    a.toks = (int32_t *)p;
+    p += up256((size_t)a.cap * 12);
+    char *state = p;
+    size_t zero = up256((size_t)a.L * a.P * 8);
+    a.h = (float *)p;
+    a.hw = (uint64_t *)p;
+    p += zero;
+    a.c = (float *)p;
+    a.gpw = (uint64_t *)p;
+    if (res) {
+        a.jw = (uint64_t *)(p + up256((size_t)a.J * 8));
+        zero += up256((size_t)a.J * 8) + up256((size_t)2 * kJointWords * 8);
+    } else {
+        zero += up256((size_t)a.L * a.P * 4);
+        p += up256((size_t)a.L * a.P * 4);
+        a.gp = (float *)p;
+        a.logit = (float *)(p + up256((size_t)a.J * 4));
+    }
+    /* the arrivals, the flag, the counts and the state (or the words' step
+     * numbers) start at zero (c and h: the reference zeroes them a segment,
+     * core/decoder.c:158-165); the streaming kernel's logits and gp and the
+     * tokens are written before they are read */
+    if (hipMemsetAsync(a.sync, 0, 512, s) != hipSuccess || hipMemsetAsync(state, 0, zero, s) != hipSuccess)
+        return -1;
     void *args[] = { &a };
-    const void *k = res ? (const void *)search_kernel<4, kResUnits, true> : (const void *)search_kernel<4, 16, false>;
-    const hipError_t e = hipLaunchCooperativeKernel(k, dim3(G), dim3(256), args, 0, s);
+    const void *k = res ? (const void *)search_resident_kernel : (const void *)search_kernel<4, 16>;
+    const hipError_t e = hipLaunchCooperativeKernel(k, dim3(G), dim3(res ? 512 : 256), args, 0, s);
     return e == hipSuccess ? 0 : -1;
 }
 

@@ -1520,17 +1520,25 @@ int pk_hip_search_dev(const pk_hip_decoder *d, const float *f, uint32_t T, int32
     hipStream_t s = (hipStream_t)stream;
     PK_LAUNCH(pkq8::launch_search(a, ws, s), "search launch");
     g_kernel = "search";
-    uint32_t res[2] = { 0, 0 }, flag[2] = { 0, 0 };
-    PK_TRY(hipMemcpyAsync(res, a.out, sizeof res, hipMemcpyDeviceToHost, s));
-    PK_TRY(hipMemcpyAsync(flag, a.sync, sizeof flag, hipMemcpyDeviceToHost, s));
+    /* the flags and the first tokens, which follow them, in one copy */
+    constexpr uint32_t kHead = 256;
+    struct {
+        uint32_t flag[2], res[2], pad[124];
+        int32_t toks[3 * kHead];
+    } head;
+    static_assert(offsetof(decltype(head), toks) == 512, "the workspace's tokens are 512 bytes in");
+    const uint32_t nhead = cap < kHead ? cap : kHead;
+    PK_TRY(hipMemcpyAsync(&head, ws, 512 + (size_t)nhead * 12, hipMemcpyDeviceToHost, s));
     PK_TRY(hipStreamSynchronize(s));
-    if (flag[1])
+    const uint32_t *res = head.res;
+    if (head.flag[1])
         return fail(PK_HIP_ETIMEOUT, "search: a grid-wide wait ran past its %u iterations; the launch left early",
                     a.spin);
     if (res[1] == 2 || res[0] > cap)
         return fail(PK_HIP_EINVAL, "search: more than cap %u tokens", cap);
-    if (res[0])
-        PK_TRY(hipMemcpy(toks, a.toks, (size_t)res[0] * 12, hipMemcpyDeviceToHost));
+    memcpy(toks, head.toks, (size_t)(res[0] < nhead ? res[0] : nhead) * 12);
+    if (res[0] > nhead)
+        PK_TRY(hipMemcpy(toks + 3 * nhead, a.toks + 3 * nhead, (size_t)(res[0] - nhead) * 12, hipMemcpyDeviceToHost));
     *ntoks = res[0];
     return PK_HIP_OK;
 }

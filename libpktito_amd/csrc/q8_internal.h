@@ -172,9 +172,10 @@ int launch_joint(float *logit, uint32_t *tok_dur, const int8_t *w, uint64_t wstr
  * zeroes the arrivals, the flag and the state on s, and launches. 0, -2 for
  * shapes it does not take, -1 for a failed call. */
 constexpr int kMaxDecLayers = 8;
-/* the search keeps its panels resident (gate panels in registers, the
- * joint's in LDS) up to this many LSTM layers and units a panel row */
+/* the search keeps its panels resident in its workgroups' registers up to
+ * this many LSTM layers and units a panel row */
 constexpr int kResLayers = 2, kResUnits = 10;
+constexpr int kJointWords = 128 + 64;
 
 struct SearchArgs {
     const float *f;                                 /* [T][J], the joint's encoder half of each frame */
@@ -187,12 +188,17 @@ struct SearchArgs {
     uint32_t P, L, J, V, n_dur, rows_out, blank, max_symbols, T, cap, kr_p, kr_j, spin;
     int32_t dur[64];
     uint32_t *sync;                                 /* [1] the error flag, [64 + b] workgroup b's last barrier: zero at launch */
+    uint32_t *out;                                  /* [0] tokens, [1] 0, or 2 when cap was reached: sync + 2 */
+    int32_t *toks;                                  /* [cap][3]: token, frame, duration */
+    /* the streaming kernel's state */
     float *h;                                       /* [L][2][P], zero at launch */
     float *c;                                       /* [L][P], zero at launch */
     float *gp;                                      /* [J] */
     float *logit;                                   /* [rows_out] */
-    int32_t *toks;                                  /* [cap][3]: token, frame, duration */
-    uint32_t *out;                                  /* [0] tokens, [1] 0, or 2 when cap was reached */
+    /* the resident kernel's words, a value above its step's number, zero at
+     * launch: [L][P], [J], and two sets of kJointWords (128 panels' bests, 64
+     * durations' keys) */
+    uint64_t *hw, *gpw, *jw;
 };
 
 size_t search_workspace_bytes(uint32_t L, uint32_t P, uint32_t J, uint32_t rows_out, uint32_t cap);

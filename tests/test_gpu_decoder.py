@@ -319,3 +319,49 @@ def test_search_in_one_launch_other_shapes(hip, torch, P, L, J, V, durs):
     finally:
         dd.release()
     assert len(want) > 0
+
+
+@pytest.mark.parametrize("P,L,J,V,durs,mark", [(640, 2, 640, 1024, [0, 9, 20], None), (32, 1, 32, 14, [1, 3], None),
+                                               (96, 2, 640, 17, [0, 1, 2], None), (640, 1, 32, 2000, [1], None),
+                                               (64, 2, 96, 200, [0, 1, 4], "ties"), (64, 2, 96, 200, [1, 2], "nan0"),
+                                               (64, 2, 96, 200, [1, 2, 3], "nan"), (64, 2, 96, 63, [2] * 64, "zeros")])
+def test_search_resident_edges(hip, torch, P, L, J, V, durs, mark):
+    """The resident search where it can go wrong: steps past the frames it
+    holds ahead and back to the same one, workgroups without units, without a
+    jpred or without a jout panel, one panel of everything, frames off
+    16-byte alignment, 64 durations, and logits placed by jout's biases:
+    equal ones (the first wins, across panels too), a NaN at token 0 and at
+    the first duration, NaNs elsewhere, zeros of both signs."""
+    dec = synth.decoder_weights(synth.rng(P + J + V), P=P, L=L, J=J, V=V, n_dur=len(durs))
+    b = dec["jout_b"]
+    if mark == "ties":
+        dec["jout_s"][:] = 0
+        b[:V + 1 + len(durs)] = 0.5
+        b[[40, 41, 90, 180]] = 7.0
+    elif mark == "nan0":
+        b[[0, V + 1]] = np.nan
+    elif mark == "nan":
+        b[[3, 17, V + 2]] = np.nan
+    elif mark == "zeros":
+        dec["jout_s"][:] = 0
+        b[:V + 1 + len(durs)] = np.where(np.arange(V + 1 + len(durs)) % 2, 0.0, -0.0)
+    T, blank = 70, V
+    frames = (synth.rng(P + 1).standard_normal((T, J)) * 2.0).astype(np.float32)
+    dw = ol.DecoderWeights(dec)
+    st = {"h": np.zeros((L, P), np.float32), "c": np.zeros((L, P), np.float32), "gp": None}
+
+    def o_predict(k):
+        st["h"], st["c"], st["gp"] = ol.predict(dw, k, st["h"], st["c"])
+
+    def o_joint(t):
+        _, k, di = ol.joint(dw, frames[t], st["gp"])
+        return k, di
+    want = search(T, o_predict, o_joint, blank, durs, 3)
+    dd = hip.DeviceDecoder(dec, torch)
+    try:
+        fd = dev(torch, np.concatenate([np.zeros(1, np.float32), frames.reshape(-1)]))
+        say("resident search", P, L, J, V, len(durs), mark)
+        got = dd.search(None, T, blank, durs, 3, f_ptr=fd.data_ptr() + 4)
+    finally:
+        dd.release()
+    assert got == want and len(want) > 0
