@@ -1183,7 +1183,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs &g, const Seg &sg, uint
     static_assert(SLOTU % NW == 0, "each wave loads whole units");
     constexpr int L = SLOTU / NW;
     constexpr int BPU = BLK == 2 ? 2 : 1, BPS = BLK ? BPU * UPS : 0;     /* blocks a unit, a stage */
-    static_assert(BLK == 0 || (KG == 1 && BM % 64 == 0), "blocks: one K group, whole 64-frame chunks");
+    static_assert(BLK == 0 || (KG == 1 && BM * BPS % 64 == 0), "blocks: one K group, whole 64-scale chunks");
     constexpr int DCH = BLK ? BM * BPS / 64 : 0;                          /* 64-float chunks of d a stage */
     constexpr int LD = (DCH + NW - 1) / NW, LT = L + LD;                  /* loads a wave issues a stage */
     static_assert(NS >= 2 && NS <= 8, "two to eight slots");
@@ -1254,18 +1254,18 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs &g, const Seg &sg, uint
             __builtin_amdgcn_global_load_lds(PK_AS1(gp), PK_AS3(slot + (wave * L + s) * kUnitBytes), 16, 0, 0);
         }
         if constexpr (BLK != 0) {
-            /* chunk c: block c / (BM / 64) of the stage, frames (c % (BM / 64)) * 64 + lane;
-             * a wave past the last chunk loads the last one again (the same bytes) */
+            /* chunk c: scales 64 c + lane of the stage's [block][frame]; a wave
+             * past the last chunk loads the last one again (the same bytes) */
 #pragma unroll
             for (int i = 0; i < LD; i++) {
                 const int c = wave + NW * i < DCH ? wave + NW * i : DCH - 1;
-                const int blk = c / (BM / 64), fc = c % (BM / 64);
-                uint32_t f = m0 + fc * 64 + lane;
+                const int blk = (c * 64 + lane) / BM;
+                uint32_t f = m0 + (c * 64 + lane) % BM;
                 f = f < T ? f : T - 1;
                 uint32_t bi = (u0 + j * UPS) * BPU + blk;
                 bi = bi < nb ? bi : nb - 1;
                 __builtin_amdgcn_global_load_lds(PK_AS1(sg.d + (size_t)f * nb + bi),
-                                                 PK_AS3(slot + SLOTU * kUnitBytes + (blk * BM + fc * 64) * 4), 4, 0, 0);
+                                                 PK_AS3(slot + SLOTU * kUnitBytes + c * 256), 4, 0, 0);
             }
         }
     };
@@ -1893,6 +1893,9 @@ struct RingCfg {
     void (*run32)(const GemmArgs &, const SegTable &, hipStream_t);   /* blocks of 32 inputs, or null */
     void (*batch64)(const JobTable &, hipStream_t);                   /* batches in blocks of 64, or null */
     void (*batch32)(const JobTable &, hipStream_t);                   /* batches in blocks of 32, or null */
+    /* whether the blocked builds have the fused SiLU quantize: pipe_tile with
+     * two channel waves of 32 (WN == 2 and TN == 2) */
+    bool silu;
 };
 static const RingCfg kRing[] = {
     /* ring_tile: name <channels x frames, units a stage> */
@@ -1902,9 +1905,9 @@ static const RingCfg kRing[] = {
     { "ring<64x64,4>", 64, 64, 4, 0, 1, run_ring<2, 2, 2, 2, 4>, nullptr, nullptr, nullptr },
     /* pipe_tile: name <channels x frames, units a stage, slots>; w8: eight
      * waves of 64 x 32 */
-    { "pipe<128x128,1,4>", 128, 128, 1, 4, 1, run_pipe<2, 2, 4, 4, 1, 4, 1>, run_pipe_batch<2, 2, 4, 4, 1, 4, 1>, run_pipe<2, 2, 4, 4, 1, 4, 1, 1>, run_pipe<2, 2, 4, 4, 1, 4, 1, 2>, run_pipe_batch<2, 2, 4, 4, 1, 4, 1, 1>, run_pipe_batch<2, 2, 4, 4, 1, 4, 1, 2> },
-    { "pipe<128x128w8,1,4>", 128, 128, 1, 4, 1, run_pipe<2, 4, 4, 2, 1, 4, 1>, run_pipe_batch<2, 4, 4, 2, 1, 4, 1>, run_pipe<2, 4, 4, 2, 1, 4, 1, 1>, run_pipe<2, 4, 4, 2, 1, 4, 1, 2>, run_pipe_batch<2, 4, 4, 2, 1, 4, 1, 1>, run_pipe_batch<2, 4, 4, 2, 1, 4, 1, 2> },
-    { "pipe<64x64,2,4>", 64, 64, 2, 4, 1, run_pipe<2, 2, 2, 2, 2, 4, 1>, run_pipe_batch<2, 2, 2, 2, 2, 4, 1>, run_pipe<2, 2, 2, 2, 2, 4, 1, 1>, run_pipe<2, 2, 2, 2, 2, 4, 1, 2>, run_pipe_batch<2, 2, 2, 2, 2, 4, 1, 1>, run_pipe_batch<2, 2, 2, 2, 2, 4, 1, 2> },
+    { "pipe<128x128,1,4>", 128, 128, 1, 4, 1, run_pipe<2, 2, 4, 4, 1, 4, 1>, run_pipe_batch<2, 2, 4, 4, 1, 4, 1>, run_pipe<2, 2, 4, 4, 1, 4, 1, 1>, run_pipe<2, 2, 4, 4, 1, 4, 1, 2>, run_pipe_batch<2, 2, 4, 4, 1, 4, 1, 1>, run_pipe_batch<2, 2, 4, 4, 1, 4, 1, 2>, false },
+    { "pipe<128x128w8,1,4>", 128, 128, 1, 4, 1, run_pipe<2, 4, 4, 2, 1, 4, 1>, run_pipe_batch<2, 4, 4, 2, 1, 4, 1>, run_pipe<2, 4, 4, 2, 1, 4, 1, 1>, run_pipe<2, 4, 4, 2, 1, 4, 1, 2>, run_pipe_batch<2, 4, 4, 2, 1, 4, 1, 1>, run_pipe_batch<2, 4, 4, 2, 1, 4, 1, 2>, false },
+    { "pipe<64x64,2,4>", 64, 64, 2, 4, 1, run_pipe<2, 2, 2, 2, 2, 4, 1>, run_pipe_batch<2, 2, 2, 2, 2, 4, 1>, run_pipe<2, 2, 2, 2, 2, 4, 1, 1>, run_pipe<2, 2, 2, 2, 2, 4, 1, 2>, run_pipe_batch<2, 2, 2, 2, 2, 4, 1, 1>, run_pipe_batch<2, 2, 2, 2, 2, 4, 1, 2>, true },
     { "pipe<64x64,4,4>", 64, 64, 4, 4, 1, run_pipe<2, 2, 2, 2, 4, 4, 1>, run_pipe_batch<2, 2, 2, 2, 4, 4, 1>, nullptr, nullptr },
     /* eight waves of 64 x 64 */
     { "pipe<128x256w8,1,4>", 128, 256, 1, 4, 1, run_pipe<2, 4, 4, 4, 1, 4, 1>, run_pipe_batch<2, 4, 4, 4, 1, 4, 1>, nullptr, nullptr },
@@ -1917,12 +1920,18 @@ static const RingCfg kRing[] = {
     { "pipe<64x64,1,4,k2>", 64, 64, 1, 4, 2, run_pipe<2, 2, 2, 2, 1, 4, 2>, run_pipe_batch<2, 2, 2, 2, 1, 4, 2>, nullptr, nullptr },
     { "pipe<64x64,2,2,k2>", 64, 64, 2, 2, 2, run_pipe<2, 2, 2, 2, 2, 2, 2>, run_pipe_batch<2, 2, 2, 2, 2, 2, 2>, nullptr, nullptr },
     /* three slots: three workgroups a CU */
-    { "pipe<64x64,2,3>", 64, 64, 2, 3, 1, run_pipe<2, 2, 2, 2, 2, 3, 1>, run_pipe_batch<2, 2, 2, 2, 2, 3, 1>, run_pipe<2, 2, 2, 2, 2, 3, 1, 1>, run_pipe<2, 2, 2, 2, 2, 3, 1, 2>, run_pipe_batch<2, 2, 2, 2, 2, 3, 1, 1>, run_pipe_batch<2, 2, 2, 2, 2, 3, 1, 2> },
+    { "pipe<64x64,2,3>", 64, 64, 2, 3, 1, run_pipe<2, 2, 2, 2, 2, 3, 1>, run_pipe_batch<2, 2, 2, 2, 2, 3, 1>, run_pipe<2, 2, 2, 2, 2, 3, 1, 1>, run_pipe<2, 2, 2, 2, 2, 3, 1, 2>, run_pipe_batch<2, 2, 2, 2, 2, 3, 1, 1>, run_pipe_batch<2, 2, 2, 2, 2, 3, 1, 2>, true },
     { "pipe<64x64,2,3,k2>", 64, 64, 2, 3, 2, run_pipe<2, 2, 2, 2, 2, 3, 2>, run_pipe_batch<2, 2, 2, 2, 2, 3, 2>, nullptr, nullptr },
     /* eight waves of 32 x 16: two a SIMD, so one wave's block chain runs
      * beside the other's MFMAs where a product has too few tiles for two
      * workgroups a CU */
-    { "pipe<64x64w8,2,4>", 64, 64, 2, 4, 1, run_pipe<2, 4, 2, 1, 2, 4, 1>, run_pipe_batch<2, 4, 2, 1, 2, 4, 1>, run_pipe<2, 4, 2, 1, 2, 4, 1, 1>, run_pipe<2, 4, 2, 1, 2, 4, 1, 2>, run_pipe_batch<2, 4, 2, 1, 2, 4, 1, 1>, run_pipe_batch<2, 4, 2, 1, 2, 4, 1, 2> },
+    { "pipe<64x64w8,2,4>", 64, 64, 2, 4, 1, run_pipe<2, 4, 2, 1, 2, 4, 1>, run_pipe_batch<2, 4, 2, 1, 2, 4, 1>, run_pipe<2, 4, 2, 1, 2, 4, 1, 1>, run_pipe<2, 4, 2, 1, 2, 4, 1, 2>, run_pipe_batch<2, 4, 2, 1, 2, 4, 1, 1>, run_pipe_batch<2, 4, 2, 1, 2, 4, 1, 2>, true },
+    /* four waves of 16 x 16, long stages: two of them a CU, for products
+     * whose 64 x 64 tiles would leave most of the chip idle (one wave's pass
+     * over K takes a tile's time however few the tiles) */
+    { "pipe<32x32,4,4>", 32, 32, 4, 4, 1, run_pipe<2, 2, 1, 1, 4, 4, 1>, run_pipe_batch<2, 2, 1, 1, 4, 4, 1>, run_pipe<2, 2, 1, 1, 4, 4, 1, 1>, run_pipe<2, 2, 1, 1, 4, 4, 1, 2>, run_pipe_batch<2, 2, 1, 1, 4, 4, 1, 1>, run_pipe_batch<2, 2, 1, 1, 4, 4, 1, 2>, false },
+    /* four waves of 32 x 16 */
+    { "pipe<64x32,2,3>", 64, 32, 2, 3, 1, run_pipe<2, 2, 2, 1, 2, 3, 1>, run_pipe_batch<2, 2, 2, 1, 2, 3, 1>, run_pipe<2, 2, 2, 1, 2, 3, 1, 1>, run_pipe<2, 2, 2, 1, 2, 3, 1, 2>, run_pipe_batch<2, 2, 2, 1, 2, 3, 1, 1>, run_pipe_batch<2, 2, 2, 1, 2, 3, 1, 2>, true },
 };
 constexpr int kNRing = sizeof kRing / sizeof kRing[0];
 
@@ -1972,23 +1981,31 @@ static int pick_ring(uint32_t rows, uint64_t frames, uint32_t ku) {
     if (g_forced_ring >= 0 && fits(g_forced_ring, ku))
         return g_forced_ring;
     auto tiles = [&](int i) { return (uint64_t)((rows + kRing[i].bn - 1) / kRing[i].bn) * ((frames + kRing[i].bm - 1) / kRing[i].bm); };
-    static const int w8 = ring_index("pipe<64x64w8,2,4>"), s3 = ring_index("pipe<64x64,2,3>");
-    /* measured on the layer's shapes at 750 and 7500 frames (every tiling,
+    static const int w8 = ring_index("pipe<64x64w8,2,4>"), s3 = ring_index("pipe<64x64,2,3>"),
+                     small = ring_index("pipe<32x32,4,4>");
+    /* measured on the layer's shapes from 20 to 7500 frames (every tiling,
      * every product): a CU's worth of 128 x 128 tiles takes the eight-wave
-     * pipelined tile; fewer take 64 x 64 pipelined tiles of two-unit stages:
-     * split into two K groups where the inputs are deep; eight waves of
-     * 32 x 16 (two a SIMD) where the tiles leave CUs idle; three slots
-     * (three workgroups a CU) where there are two tiles a CU or more;
-     * inputs too short for their slots take the ring, 64 x 64, with longer
-     * stages the fewer the tiles */
+     * pipelined tile; where two 32 x 32 tiles a CU hold the whole product,
+     * those (us, 32 x 32 against the best 64 x 64: 1024 -> 1024 at 100 frames
+     * 3.2 against 4.1, at 384 4.1 against 4.3, at 750, where they are three a
+     * CU, 5.1 against 4.8; 4096 -> 1024 at 100 frames 6.0 against 8.5, at 384
+     * 8.0 against 8.8; 1024 -> 640 at 750 4.0 against 4.5); more take 64 x 64
+     * pipelined tiles of two-unit stages: split into two K groups where the
+     * inputs are deep; eight waves of 32 x 16 (two a SIMD) below two tiles a
+     * CU (1024 -> 4096 at 384 frames 6.5 against 7.0 us with four waves);
+     * three slots (three workgroups a CU) from there on; inputs too short for
+     * their slots take the ring, 64 x 64, with longer stages the fewer the
+     * tiles */
     if (tiles(0) >= 256 && fits(5, ku))
         return 5;
+    if (tiles(small) <= 512 && fits(small, ku))
+        return small;
     if (ku >= 32 && tiles(6) < 512 && fits(13, ku))
         return 13;          /* deep inputs, few tiles: two K groups a tile */
     const uint64_t t64 = tiles(1);
-    if (t64 < 256 && w8 >= 0 && fits(w8, ku))
+    if (t64 < 512 && fits(w8, ku))
         return w8;
-    if (t64 >= 512 && s3 >= 0 && fits(s3, ku))
+    if (t64 >= 512 && fits(s3, ku))
         return s3;
     if (fits(6, ku))
         return 6;
@@ -1999,15 +2016,41 @@ static int pick_ring(uint32_t rows, uint64_t frames, uint32_t ku) {
     return ku % 16 == 0 ? 3 : ku % 8 == 0 ? 2 : 1;
 }
 
-/* The tile for a blocked product: the per-column pick, but deep inputs with
- * few tiles take the eight-wave tile (the two-K-group tiles have no blocked
- * build; measured in blocks of 32 and 64 at 750 frames). */
-static int pick_blocked(uint32_t rows, uint64_t frames, uint32_t ku) {
-    static const int w8 = ring_index("pipe<64x64w8,2,4>");
-    const int c = pick_ring(rows, frames, ku);
-    if (g_forced_ring < 0 && c == 13 && w8 >= 0 && fits(w8, ku))
-        return w8;
-    return c;
+/* The tile for a product in blocks of qb = 32 or 64 inputs, whose time is
+ * the blocks' float chains (VALU) and each wave's pass over K more than the
+ * loads, so more and smaller tiles pay further than above. Measured (us) on
+ * the layer's shapes from 20 to 7500 frames, every tiling:
+ *   two 32 x 32 tiles a CU at most: those (blocks of 32, 4096 -> 1024 at 384
+ *   frames 13.8 against 18.8 with 64 x 64, at 500 14.6 against 18.8, at 750,
+ *   three a CU, 22 against 19.4; 1024 -> 1024 at 137 4.8 against 7.0);
+ *   up to a 64 x 64 tile a CU: eight waves (1024 -> 2048 at 500, 256 tiles,
+ *   7.8 against 8.8 with four waves);
+ *   below two 64 x 64 tiles a CU: in blocks of 32 64 x 32 (1024 -> 4096 at
+ *   384 10.4 against 11.4), in blocks of 64, whose chains are half as long,
+ *   64 x 64 with three slots (8.8 against 9.4 with 64 x 32), four where the
+ *   inputs are deep (4096 -> 1024 at 1200 19.9 against 21.6);
+ *   more: 64 x 64 with three slots, or 128 x 128 where whole rounds of one a
+ *   CU are at least nine tenths full (1024 -> 4096 in blocks of 64 at 3000
+ *   frames, 768 tiles, 30.6 against 34.8; at 2200, 576, 28.6 against 27.7, in
+ *   blocks of 32 44.6 against 34.9). */
+static int pick_blocked(uint32_t rows, uint64_t frames, uint32_t ku, uint32_t qb) {
+    if (g_forced_ring >= 0 && fits(g_forced_ring, ku))
+        return g_forced_ring;
+    auto tiles = [&](int i) { return (uint64_t)((rows + kRing[i].bn - 1) / kRing[i].bn) * ((frames + kRing[i].bm - 1) / kRing[i].bm); };
+    static const int w8 = ring_index("pipe<64x64w8,2,4>"), s3 = ring_index("pipe<64x64,2,3>"),
+                     s4 = ring_index("pipe<64x64,2,4>"), small = ring_index("pipe<32x32,4,4>"),
+                     half = ring_index("pipe<64x32,2,3>"), big = ring_index("pipe<128x128w8,1,4>");
+    const uint64_t t128 = tiles(big), t64 = tiles(s3);
+    int c = s3;
+    if (tiles(small) <= 512 && fits(small, ku))
+        c = small;
+    else if (t64 <= 256)
+        c = w8;
+    else if (t64 < 512)
+        c = qb == 32 ? half : ku >= 32 ? s4 : s3;
+    else if (10 * t128 >= 9 * ((t128 + 255) / 256 * 256))
+        c = big;
+    return fits(c, ku) ? c : fits(s4, ku) ? s4 : 4;     /* 4 takes any ku: one unit a stage, four slots */
 }
 
 /* whether streamed tiling i (an index of kStream) takes ku units a panel: a
@@ -2158,15 +2201,15 @@ int launch_gemm(const GemmArgs &ga, const SegTable &tab, hipStream_t s, const ch
     /* blocks of 64 or 32 inputs (the encoder's modes): the pipelined tile
      * the heuristic picks for these frames, if it has a blocked variant */
     if ((mode == 1 && g.qb == 64) || (mode == 2 && g.qb == 32)) {
-        int c = pick_blocked(g.rows, frames, g.ku);
+        int c = pick_blocked(g.rows, frames, g.ku, g.qb);
         if (!(mode == 1 ? kRing[c].run64 : kRing[c].run32))
-            c = fits(6, g.ku) ? 6 : 4;      /* 4 takes any ku: one unit a stage, four slots */
-        if (g.oqp && (kRing[c].bn != 64 || kRing[c].bm != 64 || kRing[c].slots == 0 || kRing[c].kg != 1)) {
-            /* the fused epilogue is the 64 x 64 pipelined tiles' (two channel
-             * waves of 32) */
-            if (!fits(6, g.ku))
+            c = fits(6, g.ku) ? 6 : 4;      /* a forced tiling without blocks */
+        if (g.oqp && !kRing[c].silu) {
+            /* the fused epilogue is the tiles' of two channel waves of 32 */
+            static const int half = ring_index("pipe<64x32,2,3>");
+            c = kRing[c].bn < 64 && fits(half, g.ku) ? half : 6;
+            if (!fits(c, g.ku))
                 return -3;
-            c = 6;
         }
         auto run = mode == 1 ? kRing[c].run64 : kRing[c].run32;
         if (run) {
@@ -2219,7 +2262,7 @@ int launch_gemm_batch(const JobTable &jobs_in, hipStream_t s, const char **name)
             return hipPeekAtLastError() == hipSuccess ? 0 : -1;
         }
     }
-    const int c = mode == 0 ? pick_ring(rows, frames, g0.ku) : pick_blocked(rows, frames, g0.ku);
+    const int c = mode == 0 ? pick_ring(rows, frames, g0.ku) : pick_blocked(rows, frames, g0.ku, g0.qb);
     auto batch = mode == 0 ? kRing[c].batch : mode == 1 ? kRing[c].batch64 : mode == 2 ? kRing[c].batch32 : nullptr;
     if (batch) {
         batch(jobs, s);
