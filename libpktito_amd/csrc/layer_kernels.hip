@@ -781,6 +781,327 @@ __global__ __launch_bounds__(256) void att_pv_mfma_kernel(float *__restrict__ of
     }
 }
 
+/* ---------------------------------------------- attention in one kernel --
+ *
+ * The whole of a head's attention for 16 queries in one workgroup of NW
+ * waves, its 16 x T scores in LDS from the first product to the last, on
+ * 16x16x1_4b (a wave 16 queries x 64 columns, one step a dimension or key):
+ *   content  wave w takes key blocks w, w + NW, ... of 64; A = q + u (the
+ *            DK dimensions of the lane's query in registers), B = the keys;
+ *   band     the same over blocks of the T + 15 position rows m the 16
+ *            queries reach, from m = T - 1 - (i0 + 15): the sum of (i, m) is
+ *            added to the score (i, j), j = m - (T - 1) + i, each (i, j) once;
+ *   softmax  16 lanes a row as the kernels above, e left in LDS;
+ *   PV       DK / 64 waves, 64 dimensions each: A = e * (1 / sum) (the
+ *            reference's x[i] * inv, one rounding), B = 64 consecutive floats
+ *            of a key's value row, straight from memory; exactly the T keys.
+ * Every output is the same chain as the separate kernels'. The rows of y
+ * (keys, positions) come 16 dimensions at a time, a row's 64 bytes from four
+ * lanes, and turn to one row a lane through 4 KB of LDS of the wave's own
+ * (no barrier; 16-byte chunk c of row r at 4 r + (c ^ (r / 4) % 4): writes
+ * and reads both free of bank conflicts), two chunks ahead in registers and
+ * one in LDS. Workgroup b is head b % H: with 8 heads a head's keys,
+ * positions and values stay in one XCD's L2.
+ *
+ * The two products' chains are dependent MFMAs, 32 clocks each when nothing
+ * stands between them and 52 when something does, so a wave issues a chunk's
+ * 16 in a row and its LDS and memory operations between chunks. Measured, 384
+ * frames (a workgroup a CU, eight waves), clocks: content 16500 (8192 its
+ * MFMAs alone), band 16600, softmax 5100, PV 20600 (12300). The separate
+ * kernels' scores went through memory five times. */
+constexpr int kFQ = 16;                     /* queries a workgroup */
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+/* what a wave's lanes wrote to LDS before, its lanes read after (and the
+ * other way round): LDS operations of a wave run in order, so this only
+ * keeps the compiler from moving them */
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+/* an LDS row of scores: whole blocks of 64, and 20 floats that put the 16
+ * rows' 16-byte reads and four rows' 16 consecutive floats in distinct banks */
+__host__ __device__ constexpr uint32_t att_row(uint32_t T) { return ((T + 63) & ~63u) + 20; }
+
+template <int DK, int NW>
+__global__ __launch_bounds__(64 * NW, 8 / NW) void att_fused_kernel(float *__restrict__ of, const float *__restrict__ qf,
+                                                                  const float *__restrict__ kf,
+                                                                  const float *__restrict__ vf,
+                                                                  const float *__restrict__ pf,
+                                                                  const float *__restrict__ bu,
+                                                                  const float *__restrict__ bv, uint32_t T, uint32_t D,
+                                                                  uint32_t H, float scale, int8_t *__restrict__ qp,
+                                                                  float *__restrict__ qd, uint32_t qb) {
+    constexpr int NC = DK / 16;             /* chunks of 16 dimensions */
+    static_assert(NC % 2 == 0 && DK / 64 <= NW, "chunks in pairs, a wave a 64 dimensions of PV");
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t h = blockIdx.x % H, tile = blockIdx.x / H, i0 = tile * kFQ, col = h * DK, Ts = att_row(T);
+    constexpr int QS = DK + 4;              /* a query's row in LDS: 16-byte reads of 16 rows in distinct banks */
+    float *S = lds + NW * 1024;             /* [16][Ts] */
+    float *sq = S + kFQ * Ts;               /* [16][QS] */
+    float *turn = lds + wv * 1024;
+    for (int t = tid; t < kFQ * DK / 4; t += 64 * NW)
+        *(v4f *)(sq + t / (DK / 4) * QS + t % (DK / 4) * 4) =
+            *(const v4f *)(qf + (size_t)min(i0 + t / (DK / 4), T - 1) * D + col + t % (DK / 4) * 4);
+    __syncthreads();
+    const int sub = 4 * (lane >> 4), cl = lane & 15;
+
+    /* blocks of 64 rows of y against the queries with one bias: out(b, acc)
+     * takes block b's sums, row0 the row of block 0's first (rows clamped) */
+    auto product = [&](const float *__restrict__ yf, const float *__restrict__ bias, int64_t row0, uint32_t rows,
+                       uint32_t blocks, auto out) {
+        if ((uint32_t)wv >= blocks)
+            return;
+        /* a lane's four rows of a block: 16 k + lane / 4, its 16 bytes lane % 4 */
+        const float *src0, *src1, *src2, *src3;
+        auto rows_of = [&](uint32_t b) {
+            auto at = [&](int k) {
+                int64_t r = row0 + 64 * (int64_t)b + 16 * k + (lane >> 2);
+                r = r < 0 ? 0 : r >= (int64_t)rows ? rows - 1 : r;
+                return yf + (size_t)r * D + col + 4 * (lane & 3);
+            };
+            src0 = at(0), src1 = at(1), src2 = at(2), src3 = at(3);
+        };
+        struct Four {
+            v4f a, b, c, d;
+        };
+        auto load = [&](int c) {
+            return Four{ *(const v4f *)(src0 + 16 * c), *(const v4f *)(src1 + 16 * c), *(const v4f *)(src2 + 16 * c),
+                         *(const v4f *)(src3 + 16 * c) };
+        };
+        const int wr = 16 * (lane >> 2) + 4 * ((lane & 3) ^ ((lane >> 4) & 3)), key = (lane >> 2) & 3;
+        auto turned = [&](const Four &v) {
+            *(v4f *)(turn + wr) = v.a;              /* rows 16 k + lane / 4: (r / 4) % 4 is lane / 16 % 4 for every k */
+            *(v4f *)(turn + wr + 256) = v.b;
+            *(v4f *)(turn + wr + 512) = v.c;
+            *(v4f *)(turn + wr + 768) = v.d;
+            wave_sync();
+            const float *o = turn + 16 * lane;
+            const Four f{ *(const v4f *)(o + 4 * (0 ^ key)), *(const v4f *)(o + 4 * (1 ^ key)),
+                          *(const v4f *)(o + 4 * (2 ^ key)), *(const v4f *)(o + 4 * (3 ^ key)) };
+            wave_sync();
+            return f;
+        };
+        rows_of(wv);
+        Four g0 = load(0), g1 = load(1), y0, y1;
+        v4f a[DK / 4];
+#pragma unroll
+        for (int k = 0; k < DK / 4; k++)
+            a[k] = *(const v4f *)(sq + cl * QS + 4 * k) + *(const v4f *)(bias + col + 4 * k);
+        y0 = turned(g0);
+        g0 = load(2);
+        for (uint32_t b = wv; b < blocks; b += NW) {
+            v16f acc;
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                acc[r] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                /* chunk c + 1 through LDS, chunk c + 3 on its way, chunk c
+                 * multiplied (past the block: the next block's) */
+                Four &g = c % 2 ? g0 : g1;
+                (c % 2 ? y0 : y1) = turned(g);
+                if (c + 3 == NC)
+                    rows_of(b + NW < blocks ? b + NW : b);
+                g = load((c + 3) % NC);
+                /* the chunk's own products after both are under way */
+                __builtin_amdgcn_sched_barrier(0);
+                const Four &y = c % 2 ? y1 : y0;
+                auto four = [&](v4f a4, v4f b4) {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a4.x, b4.x, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a4.y, b4.y, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a4.z, b4.z, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a4.w, b4.w, acc, 0, 0, 0);
+                };
+                four(a[4 * c], y.a);
+                four(a[4 * c + 1], y.b);
+                four(a[4 * c + 2], y.c);
+                four(a[4 * c + 3], y.d);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            out(b, acc);
+        }
+    };
+
+    /* register r of a lane: query sub + r % 4, column 16 (r / 4) + cl of the block */
+    product(kf, bu, 0, T, (T + 63) / 64, [&](uint32_t b, const v16f &acc) {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            S[(sub + (r & 3)) * Ts + 64 * b + 16 * (r >> 2) + cl] = acc[r];
+    });
+    __syncthreads();
+    product(pf, bv, (int64_t)T - 1 - (i0 + kFQ - 1), 2 * T - 1, (T + kFQ - 1 + 63) / 64, [&](uint32_t b, const v16f &acc) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const uint32_t q = sub + (r & 3), j = 64 * b + 16 * (r >> 2) + cl - (kFQ - 1) + q;
+            float *at = S + q * Ts + (j < T ? j : Ts - 1);      /* no key: the row's last float, which nobody reads */
+            *at = *at + acc[r];
+        }
+    });
+    __syncthreads();
+    if (tid < 16 * kFQ) {
+        float *x = S + (tid >> 4) * Ts;
+        const uint32_t l = tid & 15;
+        float m = -INFINITY;
+#pragma unroll 8
+        for (uint32_t j = l; j < T; j += 16)
+            m = __builtin_fmaxf(m, x[j] * scale);
+        m = __builtin_fmaxf(m, __shfl_xor(m, 8, 16));
+        m = __builtin_fmaxf(m, __shfl_xor(m, 4, 16));
+        m = __builtin_fmaxf(m, __shfl_xor(m, 2, 16));
+        m = __builtin_fmaxf(m, __shfl_xor(m, 1, 16));
+        float acc = 0.0f;
+#pragma unroll 8
+        for (uint32_t j = l; j < T; j += 16) {
+            const float e = pk_expf(x[j] * scale - m);
+            x[j] = e;
+            acc += e;
+        }
+        const float r = 1.0f / lanes16_sum(acc);
+#pragma unroll 8
+        for (uint32_t j = l; j < T; j += 16)
+            x[j] = x[j] * r;
+    }
+    __syncthreads();
+    /* PV on the first or the last of the waves in turn: two workgroups of a
+     * CU then tend to different SIMDs */
+    const int pw = (tile & 1) ? wv - (NW - DK / 64) : wv;
+    if (pw < 0 || pw >= DK / 64)
+        return;
+    const float *vc = vf + col + 64 * pw + lane, *e = S + (lane & 15) * Ts;
+    v16f acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+        acc[r] = 0.0f;
+    /* 16 keys' values from key j0 on; past the last whole group the last 16
+     * keys (fewer than 16: the first), which nobody uses */
+    const uint32_t top = T < 16 ? 0 : T - 16, step = T < 16 ? 0 : D;
+    struct Keys {
+        float v[16];
+    };
+    auto vload = [&](uint32_t j0) {
+        const float *p = vc + (size_t)min(j0, top) * D;
+        Keys o;
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+            o.v[k] = p[k * step];
+        return o;
+    };
+    /* nothing between a group's products: another instruction after one
+     * costs the next, which waits for its sums, 20 of its 32 clocks more */
+    auto pv16 = [&](const Keys &o, const v4f (&pr)[4]) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const v4f p = pr[k];
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(p.x, o.v[4 * k], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(p.y, o.v[4 * k + 1], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(p.z, o.v[4 * k + 2], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(p.w, o.v[4 * k + 3], acc, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    /* four groups on their way: 2048 clocks of products */
+    v4f pa[4], pb[4];
+    auto pload = [&](v4f (&pr)[4], uint32_t j0) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            pr[k] = *(const v4f *)(e + min(j0, Ts - 20) + 4 * k);
+    };
+    /* three groups of values on their way, one of probabilities */
+    Keys v0 = vload(0), v1 = vload(16), v2 = vload(32), v3 = vload(48);
+    uint32_t j0 = 0;
+    pload(pa, 0);
+    auto next = [&](Keys &v, const v4f (&now)[4], v4f (&then)[4]) {
+        pload(then, j0 + 16);
+        pv16(v, now);
+        v = vload(j0 + 64);
+        j0 += 16;
+    };
+    while (j0 + 64 <= T) {
+        next(v0, pa, pb);
+        next(v1, pb, pa);
+        next(v2, pa, pb);
+        next(v3, pb, pa);
+    }
+    if (j0 + 16 <= T)
+        next(v0, pa, pb);
+    if (j0 + 16 <= T)
+        next(v1, pb, pa);
+    if (j0 + 16 <= T)
+        next(v2, pa, pb);
+    /* exactly the T keys: a padding step would turn a -0 sum into +0 */
+    for (; j0 < T; j0++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(e[j0], vc[(size_t)j0 * D], acc, 0, 0, 0);
+    const uint32_t c0 = col + 64 * pw;
+    if (!qp) {
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            if (i0 + sub + (r & 3) < T)
+                of[(size_t)(i0 + sub + (r & 3)) * D + c0 + 16 * (r >> 2) + cl] = acc[r];
+        return;
+    }
+    /* att_pv_mfma_kernel's epilogue: the wave's 16 frames x 64 channels are
+     * one packed unit */
+    int8_t *unit = (int8_t *)turn;
+    const uint32_t NB = D / qb, G = (T + 15) / 16;
+#pragma unroll
+    for (int s4 = 0; s4 < 4; s4++) {
+#pragma unroll
+        for (int bk = 0; bk < 2; bk++) {
+            if (qb == 64 && bk == 1)
+                continue;
+            const int g0 = 2 * bk, ng = qb == 64 ? 4 : 2;
+            int m = 0;
+#pragma unroll
+            for (int gi = 0; gi < 4; gi++)
+                if (gi < ng)
+                    m = max(m, mag_bits(acc[4 * ((g0 + gi) & 3) + s4]));
+            bool zero;
+            float dv, id;
+            block_scales((uint32_t)group_max_nonneg<16>(m), zero, dv, id);
+#pragma unroll
+            for (int gi = 0; gi < 4; gi++)
+                if (gi < ng) {
+                    const int gr = (g0 + gi) & 3;
+                    unit[in_unit(16 * gr + cl, sub + s4)] = (int8_t)(zero ? 0 : q1(acc[4 * gr + s4], id));
+                }
+            if (i0 + sub + s4 < T && cl == 0)
+                qd[(size_t)(i0 + sub + s4) * NB + (c0 + 16 * g0) / qb] = dv;
+        }
+    }
+    wave_sync();
+    *(v4i *)(qp + ((size_t)(c0 / 64) * G + tile) * kUnitBytes + 16 * lane) = *(const v4i *)(unit + 16 * lane);
+}
+
+/* the kernel's LDS for T keys and NW waves */
+static size_t att_fused_lds(uint32_t T, int NW) {
+    return ((size_t)NW * 1024 + (size_t)kFQ * att_row(T) + (size_t)kFQ * (128 + 4)) * 4;
+}
+
+/* The waves of the one-kernel attention for T frames and H heads, 0 where
+ * the separate kernels are the better ones. Measured (us, 8 heads of 128, one
+ * kernel against four): up to a workgroup a CU eight waves (137 frames 15.7
+ * against 29.1, 384 25.5 against 46.5; four waves 27.1); then four waves
+ * while two workgroups fit a CU's LDS (600 60 against 66, 750 67.5 against
+ * 81.8, 820 77 against 85); past that a CU holds one workgroup, and whole
+ * rounds of them decide: eight waves where the rounds are full and at most
+ * three (1024 109 against 118, 1499 222 against 242, but 1100, its third
+ * round nearly empty, 167 against 161, and 2000, a fourth round, 406
+ * against 367). */
+static int att_fused_waves(uint32_t T, uint32_t H) {
+    const uint64_t grid = (uint64_t)H * ((T + kFQ - 1) / kFQ), rounds = (grid + 255) / 256;
+    if (grid <= 256)
+        return att_fused_lds(T, 8) <= 160 * 1024 && T <= 1536 ? 8 : 0;
+    if (2 * att_fused_lds(T, 4) <= 160 * 1024)
+        return 4;
+    return T <= 1536 && rounds <= 3 && 100 * grid >= 95 * 256 * rounds ? 8 : 0;
+}
+
 /* --------------------------------------------------------------- dwq --
  *
  * core/encoder.c:158-176 (glu_item, dw_item): h = GLU(u) (backend/ref/
@@ -1047,6 +1368,25 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
         return -2;                                  /* no quantizing epilogue there: nothing launched */
     const uint32_t dk = D / H, Ts = att_score_stride(T), tiles = (T + kAT - 1) / kAT, rows = H * T;
     float *S = ws, *inv = ws + (size_t)rows * Ts;
+    const float scale = 1.0f / sqrtf((float)dk);
+    /* an output over the queries, keys or positions (which the separate
+     * kernels have read whole before they write it) takes those */
+    auto over = [&](const float *x, uint64_t n) { return of && of < x + n && x < of + (uint64_t)T * D; };
+    const uint64_t td = (uint64_t)T * D;
+    const bool inplace = over(qf, td) || over(kf, td) || over(pf, 2 * td - D) || over(bu, D) || over(bv, D);
+    const int waves = g_att_valu || small || dk > 128 || inplace ? 0 : att_fused_waves(T, H);
+    if (waves) {
+#define PK_FUSED(DK, NW) \
+    att_fused_kernel<DK, NW><<<H * ((T + kFQ - 1) / kFQ), 64 * NW, att_fused_lds(T, NW), s>>>( \
+        of, qf, kf, vf, pf, bu, bv, T, D, H, scale, qp, qd, qb)
+        if (dk == 128) {
+            if (waves == 4) PK_FUSED(128, 4); else PK_FUSED(128, 8);
+        } else {
+            if (waves == 4) PK_FUSED(64, 4); else PK_FUSED(64, 8);
+        }
+#undef PK_FUSED
+        return hipPeekAtLastError() == hipSuccess ? 0 : -1;
+    }
     if (small) {
         const uint64_t n = (uint64_t)H * T * T;
         att_scores_small_kernel<<<(uint32_t)((n + 255) / 256), 256, 0, s>>>(S, Ts, qf, kf, pf, bu, bv, T, D, dk);
@@ -1057,7 +1397,6 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
         att_dims_kernel<false><<<dim3((T + kSY - 1) / kSY, qt, H), 256, 0, s>>>(S, Ts, qf, kf, bu, T, D, dk);
         att_dims_kernel<true><<<dim3((T + kSQ - 1 + kSY - 1) / kSY, qt, H), 256, 0, s>>>(S, Ts, qf, pf, bv, T, D, dk);
     }
-    const float scale = 1.0f / sqrtf((float)dk);
     if (T <= 16 * 16)
         att_softmax_reg_kernel<16><<<(rows + 15) / 16, 256, 0, s>>>(S, inv, Ts, rows, T, scale);
     else if (T <= 16 * 64)

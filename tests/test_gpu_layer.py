@@ -159,6 +159,35 @@ def test_attention(hip, torch, T, D, H, valu):
     assert np.array_equal(bits(o.cpu().numpy()), bits(want))
 
 
+@pytest.mark.parametrize("T,D,H", [(1, 64, 1), (15, 128, 1), (16, 1024, 8), (31, 256, 4), (49, 512, 8), (64, 128, 1),
+                                   (130, 1024, 8), (512, 1024, 8), (513, 1024, 8), (559, 512, 8), (832, 1024, 8),
+                                   (833, 1024, 8), (1020, 1024, 8), (1499, 1024, 8), (1537, 128, 1)])
+def test_attention_paths_agree(hip, torch, T, D, H):
+    """The attention on the matrix cores (one kernel or four, by the frames,
+    the heads and whether the output lies over the queries) gives the VALU
+    kernels' bits, which test_attention holds to the oracle: tiles of
+    queries and blocks of keys with every kind of remainder, both sides of
+    each rule, and the output written over the queries."""
+    g = synth.rng(T + D)
+    q, k, v = (dev(torch, g.standard_normal((T, D)).astype(np.float32)) for _ in range(3))
+    p = dev(torch, g.standard_normal((2 * T - 1, D)).astype(np.float32))
+    u, b = (dev(torch, 0.1 * g.standard_normal(D).astype(np.float32)) for _ in range(2))
+    ws = torch.empty(hip.attention_workspace(T, H), dtype=torch.uint8, device="cuda")
+    outs = []
+    for valu, inplace in ((1, False), (0, False), (0, True)):
+        was = hip.force_attention(valu)
+        try:
+            say("attention", T, D, H, "valu" if valu else "mfma", "in place" if inplace else "")
+            x = q.clone()
+            o = x if inplace else torch.full_like(q, 7.0)
+            hip.attention_dev(o, x, k, v, p, u, b, T, D, H, ws)
+            torch.cuda.synchronize()
+            outs.append(o.cpu().numpy().view(np.uint32))
+        finally:
+            hip.force_attention(was)
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+
+
 @pytest.mark.parametrize("T", [37, 301])
 @pytest.mark.parametrize("valu", [0, 1])
 def test_attention_special_values(hip, torch, valu, T):
