@@ -312,11 +312,25 @@ def _dptr(t):
     return t.data_ptr() if t is not None else None
 
 
+_current_stream = None
+
+
 def _stream(stream):
-    if stream is None:
+    """The stream handle to launch on: the caller's, or torch's current one
+    (asked for by handle where torch has that call: 0.2 us against 3.0 for
+    torch.cuda.current_stream(), a third of a small call's host time)."""
+    global _current_stream
+    if stream is not None:
+        return stream
+    if _current_stream is None:
         import torch
-        return torch.cuda.current_stream().cuda_stream
-    return stream
+        torch.cuda.current_stream()                     # torch's own initialisation and its errors
+        raw, dev = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+        if raw is not None and dev is not None:
+            _current_stream = lambda: raw(dev())
+        else:
+            _current_stream = lambda: torch.cuda.current_stream().cuda_stream
+    return _current_stream()
 
 
 def quantize_dev(q, d, x, n, qb, T, xs, stream=None):

@@ -601,3 +601,22 @@ def test_streamed_tiles_walk_every_tile(hip, torch, M, K, N, add, pad):
     assert np.array_equal(bits(ref[frames, :N]), bits(want))
     for key, o in outs.items():
         assert np.array_equal(bits(o), bits(ref)), (names[key[0]], key[1])
+
+
+def test_default_stream_is_torchs_current_one(hip, torch):
+    """Calls without a stream go to torch's current stream: the default one,
+    the one of a stream context, another thread's own, and back."""
+    import threading
+    seen = {}
+
+    def ask(key):
+        seen[key] = (hip._stream(None), torch.cuda.current_stream().cuda_stream)
+    ask("default")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        ask("context")
+        t = threading.Thread(target=ask, args=("thread",))
+        t.start()
+        t.join()
+    ask("after")
+    assert all(a == b for a, b in seen.values()) and seen["context"][0] == s.cuda_stream != seen["default"][0]
