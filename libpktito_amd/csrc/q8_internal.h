@@ -243,7 +243,8 @@ struct StreamCfg {
     const char *name;
     uint32_t bn, bm, ups, slots;        /* channels x frames, units a stage, ring slots */
     void (*run)(const GemmArgs &, const SegTable &, hipStream_t);
-    void (*batch)(const JobTable &, hipStream_t);
+    void (*batch)(const JobTable &, hipStream_t);       /* packed activations */
+    void (*grouped)(const JobTable &, hipStream_t);     /* row-major ones */
 };
 const StreamCfg *stream_cfg(int i);     /* nullptr past the last */
 int stream_count();

@@ -1984,8 +1984,11 @@ static int pick_ring(uint32_t rows, uint64_t frames, uint32_t ku) {
     static const int w8 = ring_index("pipe<64x64w8,2,4>"), s3 = ring_index("pipe<64x64,2,3>"),
                      small = ring_index("pipe<32x32,4,4>");
     /* measured on the layer's shapes from 20 to 7500 frames (every tiling,
-     * every product): a CU's worth of 128 x 128 tiles takes the eight-wave
-     * pipelined tile; where two 32 x 32 tiles a CU hold the whole product,
+     * every product): 128 x 128 tiles for five eighths of the CUs or more
+     * take the eight-wave pipelined tile (160 tiles: 4096 -> 1024 at 2500
+     * frames 20.1 us against 21.6 with 64 x 64, 1024 -> 1024 9.0 against 9.0;
+     * 232: at 3600 21.9 against 29.4, 9.8 against 11.8; 1024 -> 2048 at
+     * 1600, 208 tiles, 9.6 against 11.6); where two 32 x 32 tiles a CU hold the whole product,
      * those (us, 32 x 32 against the best 64 x 64: 1024 -> 1024 at 100 frames
      * 3.2 against 4.1, at 384 4.1 against 4.3, at 750, where they are three a
      * CU, 5.1 against 4.8; 4096 -> 1024 at 100 frames 6.0 against 8.5, at 384
@@ -1996,7 +1999,7 @@ static int pick_ring(uint32_t rows, uint64_t frames, uint32_t ku) {
      * three slots (three workgroups a CU) from there on; inputs too short for
      * their slots take the ring, 64 x 64, with longer stages the fewer the
      * tiles */
-    if (tiles(0) >= 256 && fits(5, ku))
+    if (tiles(0) >= 160 && fits(5, ku))
         return 5;
     if (tiles(small) <= 512 && fits(small, ku))
         return small;
@@ -2073,8 +2076,10 @@ static bool stream_spans_fit(const GemmArgs &g, const Seg &sg) {
 
 /* The streamed tiling (an index of stream_cfg) for a per-row product of one
  * segment, or -1 for the per-launch tiles: the forced one where it fits;
- * else 256 x 128 streamed tiles where there are at least 400 of them, or 200
- * with deep inputs (4096). Measured at 7500 frames (each product alone): ff
+ * else 256 x 128 streamed tiles where there are at least 400 of them, or,
+ * with deep inputs (4096), more than one for two CUs (129: at 4210 frames, 132
+ * tiles, 27.2 us against 30.2, at 6000 30.4 against 32.8; at 3600, 116, 27.0
+ * against 21.9). Measured at 7500 frames (each product alone): ff
  * up 41-44 against 46-47 us, pw1 24.2 against 25.9, the positions' 14999
  * rows 26-30 against 28-34, ff down 32.7-34.3 against 34.2-36.1; the 236-tile
  * products with 1024 inputs (q, k, v, o, pw2) run faster on the per-launch
@@ -2098,7 +2103,7 @@ static int pick_stream(uint32_t rows, uint64_t frames, uint32_t ku, bool batch =
     const uint64_t tiles = (uint64_t)((rows + c.bn - 1) / c.bn) * ((frames + c.bm - 1) / c.bm);
     if (batch)
         return tiles >= 1024 ? i : -1;
-    return tiles >= 400 || (ku >= 64 && tiles >= 200) ? i : -1;
+    return tiles >= 400 || (ku >= 64 && tiles > 128) ? i : -1;
 }
 
 template <int WN, int WM, int TN, int TM, int MODE>
@@ -2188,6 +2193,26 @@ int launch_gemm(const GemmArgs &ga, const SegTable &tab, hipStream_t s, const ch
         const int c = pick_stream(g.rows, frames, g.ku);
         if (c >= 0) {
             stream_cfg(c)->run(g, tab, s);
+            *name = stream_cfg(c)->name;
+            return hipPeekAtLastError() == hipSuccess ? 0 : -1;
+        }
+    }
+    if (mode == 0 && tab.nseg > 1 && tab.nseg <= (uint32_t)kMaxJobs) {
+        /* the segments as a batch's jobs, one matrix: with deep inputs only
+         * (eight segments, 4210 frames: 4096 -> 1024 28.1 us against 45.6 on
+         * the per-launch tiles, 1024 -> 4096 33.7 against 33.5) */
+        bool rows = g.ku >= 64 || g_forced_ring >= kNRing;
+        for (uint32_t i = 0; i < tab.nseg; i++)
+            rows = rows && tab.s[i].qstride == 0 && stream_spans_fit(g, tab.s[i]);
+        const int c = rows ? pick_stream(g.rows, frames, g.ku) : -1;
+        if (c >= 0) {
+            JobTable t;
+            t.njobs = tab.nseg;
+            for (uint32_t i = 0; i < tab.nseg; i++) {
+                t.g[i] = g;
+                t.s[i] = tab.s[i];
+            }
+            stream_cfg(c)->grouped(t, s);
             *name = stream_cfg(c)->name;
             return hipPeekAtLastError() == hipSuccess ? 0 : -1;
         }

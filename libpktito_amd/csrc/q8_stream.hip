@@ -523,15 +523,18 @@ static void run_stream_batch(const JobTable &jobs, hipStream_t s) {
     run_stream_jobs<WN, WM, TN, TM, UPS, NS, NL, OCC>(jobs, s, true);
 }
 
-
+template <int WN, int WM, int TN, int TM, int UPS, int NS, int NL, int OCC>
+static void run_stream_grouped(const JobTable &jobs, hipStream_t s) {
+    run_stream_jobs<WN, WM, TN, TM, UPS, NS, NL, OCC>(jobs, s, false);
+}
 
 static const StreamCfg kStreamCfgs[] = {
     /* name <channels x frames, units a stage, slots, loader waves>: eight MFMA
      * waves of 64 x 64 and four loader waves, one workgroup a CU (the ring
      * and the loaders' share of the waves leave no room for a second) */
-    { "stream<256x128,2,3,l4>", 256, 128, 2, 3, run_stream<4, 2, 4, 4, 2, 3, 4, 1>, run_stream_batch<4, 2, 4, 4, 2, 3, 4, 1> },
-    { "stream<128x256,2,3,l4>", 128, 256, 2, 3, run_stream<2, 4, 4, 4, 2, 3, 4, 1>, run_stream_batch<2, 4, 4, 4, 2, 3, 4, 1> },
-    { "stream<128x256,1,4,l4>", 128, 256, 1, 4, run_stream<2, 4, 4, 4, 1, 4, 4, 1>, run_stream_batch<2, 4, 4, 4, 1, 4, 4, 1> },
+    { "stream<256x128,2,3,l4>", 256, 128, 2, 3, run_stream<4, 2, 4, 4, 2, 3, 4, 1>, run_stream_batch<4, 2, 4, 4, 2, 3, 4, 1>, run_stream_grouped<4, 2, 4, 4, 2, 3, 4, 1> },
+    { "stream<128x256,2,3,l4>", 128, 256, 2, 3, run_stream<2, 4, 4, 4, 2, 3, 4, 1>, run_stream_batch<2, 4, 4, 4, 2, 3, 4, 1>, run_stream_grouped<2, 4, 4, 4, 2, 3, 4, 1> },
+    { "stream<128x256,1,4,l4>", 128, 256, 1, 4, run_stream<2, 4, 4, 4, 1, 4, 4, 1>, run_stream_batch<2, 4, 4, 4, 1, 4, 4, 1>, run_stream_grouped<2, 4, 4, 4, 1, 4, 4, 1> },
 };
 
 const StreamCfg *stream_cfg(int i) {
