@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void norm_kernel(float *__restrict__ x, uint32
  *   o(i, d) = chain_j fmaf(v_j[d], P(i, j))  over j = 0 .. T-1 in order.
  * The reference lays K, P and V out as panels for its CPU kernel; the bits
  * depend only on each output's chain, so the products' row-major outputs
- * are read as they are. These are VALU kernels: an MFMA's sum of products
+ * are read as they are. First the VALU kernels: an MFMA's sum of products
  * rounds differently from a chain of FMAs.
  *
  * Three kernels:
