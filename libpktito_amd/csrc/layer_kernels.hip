@@ -1369,11 +1369,14 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
     const uint32_t dk = D / H, Ts = att_score_stride(T), tiles = (T + kAT - 1) / kAT, rows = H * T;
     float *S = ws, *inv = ws + (size_t)rows * Ts;
     const float scale = 1.0f / sqrtf((float)dk);
-    /* an output over the queries, keys or positions (which the separate
-     * kernels have read whole before they write it) takes those */
+    /* an output over an input takes the separate kernels: they have read the
+     * queries, keys, positions and biases whole before they write it, and up
+     * to 64 frames the values too (PV is one workgroup a 64 dimensions of a
+     * head there, which stores what it alone has read) */
     auto over = [&](const float *x, uint64_t n) { return of && of < x + n && x < of + (uint64_t)T * D; };
     const uint64_t td = (uint64_t)T * D;
-    const bool inplace = over(qf, td) || over(kf, td) || over(pf, 2 * td - D) || over(bu, D) || over(bv, D);
+    const bool inplace = over(qf, td) || over(kf, td) || over(vf, td) || over(pf, 2 * td - D) || over(bu, D) ||
+                         over(bv, D);
     const int waves = g_att_valu || small || dk > 128 || inplace ? 0 : att_fused_waves(T, H);
     if (waves) {
 #define PK_FUSED(DK, NW) \

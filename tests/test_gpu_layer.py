@@ -188,6 +188,27 @@ def test_attention_paths_agree(hip, torch, T, D, H):
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("T,D,H", [(16, 128, 1), (17, 1024, 8), (33, 256, 4), (64, 1024, 8)])
+def test_attention_over_the_values(hip, torch, T, D, H):
+    """The output written over the values, which up to 64 frames (one
+    workgroup of PV a 64 dimensions) gives the same bits as an output of its
+    own: such a call keeps to the kernels that read before they write."""
+    g = synth.rng(3 * T + D)
+    q, k, v = (dev(torch, g.standard_normal((T, D)).astype(np.float32)) for _ in range(3))
+    p = dev(torch, g.standard_normal((2 * T - 1, D)).astype(np.float32))
+    u, b = (dev(torch, 0.1 * g.standard_normal(D).astype(np.float32)) for _ in range(2))
+    ws = torch.empty(hip.attention_workspace(T, H), dtype=torch.uint8, device="cuda")
+    want = torch.full_like(q, 7.0)
+    say("attention", T, D, H)
+    hip.attention_dev(want, q, k, v, p, u, b, T, D, H, ws)
+    ws.fill_(255)
+    say("attention over the values", T, D, H)
+    hip.attention_dev(v, q, k, v, p, u, b, T, D, H, ws)
+    torch.cuda.synchronize()
+    assert torch.equal(v.view(torch.int32), want.view(torch.int32))
+    assert not bool((ws == 255).all())          # the separate kernels: their scores went through the workspace
+
+
 @pytest.mark.parametrize("T", [37, 301])
 @pytest.mark.parametrize("valu", [0, 1])
 def test_attention_special_values(hip, torch, valu, T):
