@@ -1361,7 +1361,7 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
                      int8_t *qp, float *qd, uint32_t qb) {
     if (T == 0)
         return 0;
-    if (H == 0 || D % H || (D / H) % 16 || (uint64_t)T * att_score_stride(T) >= (1ull << 32) - 1)
+    if (H == 0 || D == 0 || D % H || (D / H) % 16 || (uint64_t)T * att_score_stride(T) >= (1ull << 32) - 1)
         return -2;
     const bool small = (D / H) % 64 != 0;
     if (qp && (g_att_valu || small || !(qb == 32 || qb == 64)))

@@ -1237,8 +1237,9 @@ int pk_hip_attention_dev(float *o, const float *q, const float *k, const float *
         return e;
     if (T == 0)
         return PK_HIP_OK;
-    if (!o || !q || !k || !v || !p || !bias_u || !bias_v || !ws || H == 0 || D % H || (D / H) % 16)
-        return fail(PK_HIP_EINVAL, "attention_dev: heads of a multiple of 16 dimensions, every pointer set");
+    if (!o || !q || !k || !v || !p || !bias_u || !bias_v || !ws || H == 0 || D == 0 || D % H || (D / H) % 16)
+        return fail(PK_HIP_EINVAL, "attention_dev: D a multiple of H, heads of a multiple of 16 dimensions (16 or more), "
+                                   "every pointer set");
     if (ws_bytes < pk_hip_attention_workspace(T, H))
         return fail(PK_HIP_EINVAL, "attention_dev: workspace of %zu bytes, %zu needed", ws_bytes,
                     pk_hip_attention_workspace(T, H));
@@ -1256,8 +1257,9 @@ int pk_hip_attention_noalloc_dev(float *o, const float *q, const float *k, const
         return e;
     if (T == 0)
         return PK_HIP_OK;
-    if (!o || !q || !k || !v || !p || !bias_u || !bias_v || H == 0 || D % H || (D / H) % 16)
-        return fail(PK_HIP_EINVAL, "attention_noalloc_dev: heads of a multiple of 16 dimensions, every pointer set");
+    if (!o || !q || !k || !v || !p || !bias_u || !bias_v || H == 0 || D == 0 || D % H || (D / H) % 16)
+        return fail(PK_HIP_EINVAL, "attention_noalloc_dev: D a multiple of H, heads of a multiple of 16 dimensions (16 or more), "
+                                   "every pointer set");
     const size_t need = pk_hip_attention_workspace(T, H);
     if (need > pkq8::kStaticScratchBytes)
         return fail(PK_HIP_EINVAL,

@@ -209,6 +209,22 @@ def test_attention_over_the_values(hip, torch, T, D, H):
     assert not bool((ws == 255).all())          # the separate kernels: their scores went through the workspace
 
 
+def test_attention_refuses_heads_of_no_dimensions(hip, torch):
+    """D = 0 (or fewer dimensions than heads) is refused on the host by both
+    entries, whatever buffers come with it: nothing is launched, and the
+    output and the workspace keep their bytes."""
+    t = torch.full((64, 128), 7.0, dtype=torch.float32, device="cuda")
+    ws = torch.full((hip.attention_workspace(17, 2),), 255, dtype=torch.uint8, device="cuda")
+    for D, H in ((0, 2), (0, 1), (1, 2)):
+        for call in (lambda: hip.attention_dev(t, t, t, t, t, t, t, 17, D, H, ws),
+                     lambda: hip.attention_noalloc_dev(t, t, t, t, t, t, t, 17, D, H)):
+            with pytest.raises(hip.PkHipError) as e:
+                call()
+            assert e.value.code == hip.PK_HIP_EINVAL
+    torch.cuda.synchronize()
+    assert bool((t == 7.0).all()) and bool((ws == 255).all())
+
+
 @pytest.mark.parametrize("T", [37, 301])
 @pytest.mark.parametrize("valu", [0, 1])
 def test_attention_special_values(hip, torch, valu, T):
