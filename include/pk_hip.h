@@ -440,11 +440,12 @@ int pk_hip_force_search_resident(int on);
  * returns the one forced before. All compute the same bits. */
 int pk_hip_force_quantize(int kind);
 
-/* Tests and tuning: the attention's score and PV products for every later
- * launch in the process: 0 on the matrix cores (one-step fp32 MFMAs, the
- * default), 1 as VALU fma chains; returns the one set before. Both compute
- * the same bits. */
-int pk_hip_force_attention(int valu);
+/* Tests and tuning: the attention's kernels for every later launch in the
+ * process: 0 on the matrix cores (one-step fp32 MFMAs), in one kernel or in
+ * separate ones by size (the default), 1 as VALU fma chains, 2 on the matrix
+ * cores in separate kernels always; any other value is 1. Returns the one
+ * set before. All compute the same bits. */
+int pk_hip_force_attention(int kind);
 
 #ifdef __cplusplus
 }

@@ -240,8 +240,9 @@ def force_quantize(kind):
 
 
 def force_attention(valu):
-    """The attention's score and PV products for every later launch: 0 on
-    the matrix cores (the default), 1 as VALU fma chains; returns the one
+    """The attention's kernels for every later launch: 0 on the matrix cores,
+    in one kernel or in separate ones by size (the default), 1 as VALU fma
+    chains, 2 on the matrix cores in separate kernels always; returns the one
     set before."""
     return lib().pk_hip_force_attention(int(valu))
 

@@ -1288,13 +1288,14 @@ __global__ __launch_bounds__(256) void att_pv_small_kernel(float *__restrict__ o
     of[(size_t)i * D + d] = acc;
 }
 
-/* The attention's kernels: 0 the matrix cores' (the default), 1 the VALU
- * chains; both compute the same bits. */
-static int g_att_valu = 0;
+/* The attention's kernels: 0 the matrix cores', one kernel or separate ones
+ * by size (the default), 1 the VALU chains, 2 the matrix cores' separate
+ * ones; all compute the same bits. */
+static int g_att_kind = 0;
 
-int set_attention_kernels(int valu) {
-    const int was = g_att_valu;
-    g_att_valu = valu ? 1 : 0;
+int set_attention_kernels(int kind) {
+    const int was = g_att_kind;
+    g_att_kind = kind == 0 || kind == 2 ? kind : 1;
     return was;
 }
 
@@ -1364,7 +1365,7 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
     if (H == 0 || D == 0 || D % H || (D / H) % 16 || (uint64_t)T * att_score_stride(T) >= (1ull << 32) - 1)
         return -2;
     const bool small = (D / H) % 64 != 0;
-    if (qp && (g_att_valu || small || !(qb == 32 || qb == 64)))
+    if (qp && (g_att_kind == 1 || small || !(qb == 32 || qb == 64)))
         return -2;                                  /* no quantizing epilogue there: nothing launched */
     const uint32_t dk = D / H, Ts = att_score_stride(T), tiles = (T + kAT - 1) / kAT, rows = H * T;
     float *S = ws, *inv = ws + (size_t)rows * Ts;
@@ -1377,7 +1378,7 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
     const uint64_t td = (uint64_t)T * D;
     const bool inplace = over(qf, td) || over(kf, td) || over(vf, td) || over(pf, 2 * td - D) || over(bu, D) ||
                          over(bv, D);
-    const int waves = g_att_valu || small || dk > 128 || inplace ? 0 : att_fused_waves(T, H);
+    const int waves = g_att_kind || small || dk > 128 || inplace ? 0 : att_fused_waves(T, H);
     if (waves) {
 #define PK_FUSED(DK, NW) \
     att_fused_kernel<DK, NW><<<H * ((T + kFQ - 1) / kFQ), 64 * NW, att_fused_lds(T, NW), s>>>( \
@@ -1393,7 +1394,7 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
     if (small) {
         const uint64_t n = (uint64_t)H * T * T;
         att_scores_small_kernel<<<(uint32_t)((n + 255) / 256), 256, 0, s>>>(S, Ts, qf, kf, pf, bu, bv, T, D, dk);
-    } else if (g_att_valu) {
+    } else if (g_att_kind == 1) {
         att_scores_kernel<<<dim3(tiles, tiles, H), 256, 0, s>>>(S, Ts, qf, kf, pf, bu, bv, T, D, dk);
     } else {
         const uint32_t qt = (T + kSQ - 1) / kSQ;
@@ -1408,7 +1409,7 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
         att_softmax_kernel<<<(rows + 15) / 16, 256, 0, s>>>(S, inv, Ts, rows, T, scale);
     if (small)
         att_pv_small_kernel<<<(uint32_t)(((uint64_t)T * D + 255) / 256), 256, 0, s>>>(of, S, inv, Ts, vf, T, D, dk);
-    else if (g_att_valu)
+    else if (g_att_kind == 1)
         att_pv_kernel<<<dim3(dk / kPD, (T + kPI - 1) / kPI, H), 128, 0, s>>>(of, S, inv, Ts, vf, T, D, dk);
     else
         att_pv_mfma_kernel<<<dim3((T + 63) / 64, dk / 64, H), 256, 0, s>>>(of, S, inv, Ts, vf, T, D, dk, qp, qd,

@@ -604,7 +604,7 @@ size_t pk_hip_gemm_workspace(uint32_t rows) { return pkq8::skinny_workspace_byte
 
 int pk_hip_force_quantize(int kind) { return pkq8::set_quant_kernel(kind); }
 
-int pk_hip_force_attention(int valu) { return pkq8::set_attention_kernels(valu); }
+int pk_hip_force_attention(int kind) { return pkq8::set_attention_kernels(kind); }
 
 int pk_hip_force_search_resident(int on) { return pkq8::set_search_resident(on != 0) ? 1 : 0; }
 

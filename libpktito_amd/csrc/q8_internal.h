@@ -120,9 +120,10 @@ int set_ring(int i);
  * whole column, -1 by size; returns the one forced before. */
 int set_quant_kernel(int kind);
 
-/* The attention's score and PV kernels: 0 the matrix cores', 1 the VALU
- * chains; returns the one set before. */
-int set_attention_kernels(int valu);
+/* The attention's kernels: 0 the matrix cores', one kernel or separate ones
+ * by size, 1 the VALU chains, 2 the matrix cores' separate ones; returns the
+ * one set before. */
+int set_attention_kernels(int kind);
 
 /* The quantize's op on its inputs (launch_quantize_packed's op). */
 constexpr int kOpPlain = 0, kOpSilu = 1;

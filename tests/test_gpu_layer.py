@@ -130,7 +130,7 @@ def test_dwq(hip, torch, T, D, K, qb):
     check_packed(qp, dt, q, d, D, T)
 
 
-@pytest.mark.parametrize("valu", [0, 1])
+@pytest.mark.parametrize("valu", [0, 1, 2])
 @pytest.mark.parametrize("T,D,H", [(1, 128, 2), (2, 128, 2), (7, 64, 1), (17, 128, 2), (64, 128, 2), (65, 256, 2),
                                    (130, 128, 2), (100, 1024, 8), (289, 128, 1),
                                    (37, 64, 4), (50, 128, 4), (9, 96, 2), (300, 64, 4)])
@@ -138,9 +138,10 @@ def test_attention(hip, torch, T, D, H, valu):
     """The attention's scores (with the positions' diagonals), softmax and
     weighted values against pk_k_gemm_f32 and pk_k_softmax composed on the
     CPU with the reference's panel layouts; on the matrix cores (one-step
-    MFMAs) and as VALU chains. T covers one key, partial tiles and bands,
-    and key counts that are not multiples of 8; heads of 16, 32 and 48
-    dimensions run on the one-thread-an-output kernels."""
+    MFMAs) in one kernel (0) and in separate ones (2) and as VALU chains (1).
+    T covers one key, partial tiles and bands, and key counts that are not
+    multiples of 8; heads of 16, 32 and 48 dimensions run on the
+    one-thread-an-output kernels whatever valu."""
     g = synth.rng(T * 7 + D)
     q, k, v = (g.standard_normal((3, T, D)) * 1.5).astype(np.float32)
     p = g.standard_normal((2 * T - 1, D)).astype(np.float32)
@@ -226,12 +227,14 @@ def test_attention_refuses_heads_of_no_dimensions(hip, torch):
 
 
 @pytest.mark.parametrize("T", [37, 301])
-@pytest.mark.parametrize("valu", [0, 1])
+@pytest.mark.parametrize("valu", [0, 1, 2])
 def test_attention_special_values(hip, torch, valu, T):
     """Subnormal and signed-zero operands, products past the float range and
     NaNs in the queries, keys, values and positions: every chain step's one
     rounding (an MFMA step or a v_fma_f32) gives the oracle's bits, NaNs
-    compared as NaN. T = 301 takes the softmax kernel of rows over 256 keys."""
+    compared as NaN. In one kernel (0), as VALU chains (1) and in the matrix
+    cores' separate kernels (2); there and in the VALU's T = 301 takes the
+    softmax kernel of rows over 256 keys."""
     D, H = 128, 2
     g = synth.rng(4242)
     q, k, v = (g.standard_normal((3, T, D)) * 1.5).astype(np.float32)
@@ -302,12 +305,13 @@ def test_layer_small_heads(hip, torch, T, qb):
     run_layer(hip, torch, D=64, H=4, F=128, K=9, T=T, qb=qb, seed=900 + T)
 
 
-@pytest.mark.parametrize("valu", [0, 1])
+@pytest.mark.parametrize("valu", [0, 1, 2])
 @pytest.mark.parametrize("T,qb", [(1, 32), (2, 64), (37, 32), (100, 64)])
 def test_layer_small(hip, torch, T, qb, valu):
-    """valu 0: the attention's output quantized in the PV's epilogue; valu 1:
-    the VALU attention, its output written and quantized by a pass of its
-    own."""
+    """valu 0: the attention in one kernel, its output quantized in that
+    kernel's epilogue; valu 2: in separate kernels, quantized in the PV
+    kernel's epilogue; valu 1: the VALU attention, its output written and
+    quantized by a pass of its own."""
     was = hip.force_attention(valu)
     try:
         run_layer(hip, torch, 128, 2, 256, 9, T, qb, seed=T * 3 + qb)
@@ -329,12 +333,22 @@ def test_layer_model_shapes_at_a_minute(hip, torch, T, qb):
     run_layer(hip, torch, 1024, 8, 4096, 9, T, qb, seed=T + qb)
 
 
-@pytest.mark.parametrize("valu", [0, 1])
+@pytest.mark.parametrize("T,qb", [(840, 32), (840, 64), (1020, 32), (1020, 64)])
+def test_layer_model_heads_past_two_workgroups_a_cu(hip, torch, T, qb):
+    """Layers of the model's heads (8 of 128) past the frames whose scores
+    fit a CU's LDS twice: by default 840 frames take the attention's separate
+    matrix-core kernels with the output quantized in PV's epilogue, 1020 the
+    one kernel on eight waves."""
+    run_layer(hip, torch, 1024, 8, 256, 9, T, qb, seed=T + qb)
+
+
+@pytest.mark.parametrize("valu", [0, 1, 2])
 @pytest.mark.parametrize("qb", [32, 64])
 def test_layer_attention_output_special_values(hip, torch, valu, qb):
     """Special values reaching the attention's output, which the output
-    projection's activations quantize (on the matrix cores in PV's epilogue,
-    valu 0; by a pass of its own after the VALU attention, valu 1): v's row
+    projection's activations quantize (on the matrix cores in the epilogue of
+    the one kernel, valu 0, or of the PV kernel, valu 2; by a pass of its own
+    after the VALU attention, valu 1): v's row
     scales planted so that head 0's channel 5 is NaN for every frame, head
     1's channel 70 infinite, head 2's channels 128..159 zero and head 3's
     192..223 subnormal, their attention outputs under 2^-121. Each block

@@ -2,8 +2,9 @@
 library's static scratch, against pk_hip_attention_dev with a workspace of
 its own, bit for bit: two calls in a row on the same GPU, the second on
 fewer frames (the scratch then still holds the first call's scores past the
-second's rows, which no kernel may read), on the matrix-core kernels and the
-VALU chains; and the sizes past the scratch refused before anything runs."""
+second's rows, which no kernel may read), by default (at these sizes the one
+matrix-core kernel, which leaves the scratch alone), on the VALU chains and
+on the separate matrix-core kernels; and the sizes past the scratch refused before anything runs."""
 import sys
 
 import numpy as np
@@ -38,7 +39,7 @@ def operands(torch, T, D, seed):
     return [torch.from_numpy(a).cuda() for a in (q, k, v, p, bu, bv)]
 
 
-@pytest.mark.parametrize("valu", [0, 1])
+@pytest.mark.parametrize("valu", [0, 1, 2])
 def test_noalloc_attention_is_the_workspace_ones(hip, torch, valu):
     was = hip.force_attention(valu)
     try:
@@ -74,11 +75,21 @@ def test_noalloc_attention_refuses_sizes_past_the_scratch(hip, torch):
     torch.cuda.synchronize()
 
 
-def test_noalloc_attention_under_graph_capture(hip, torch):
+@pytest.mark.parametrize("valu", [0, 2])
+def test_noalloc_attention_under_graph_capture(hip, torch, valu):
     """The entry captured into a HIP graph (what it exists for), replayed
     several times with eager work of the library between replays and new
     inputs copied in before each: every replay's output is
-    pk_hip_attention_dev's on the same inputs, bit for bit."""
+    pk_hip_attention_dev's on the same inputs, bit for bit; on the one kernel
+    (0) and on the separate kernels (2), whose scores the scratch holds."""
+    was = hip.force_attention(valu)
+    try:
+        capture_and_replay(hip, torch)
+    finally:
+        hip.force_attention(was)
+
+
+def capture_and_replay(hip, torch):
     T, D, H = 300, 512, 8
     ops = operands(torch, T, D, 77)
     ws = torch.empty((hip.attention_workspace(T, H),), dtype=torch.uint8, device="cuda")
