@@ -2019,41 +2019,75 @@ static int pick_ring(uint32_t rows, uint64_t frames, uint32_t ku) {
     return ku % 16 == 0 ? 3 : ku % 8 == 0 ? 2 : 1;
 }
 
+/* What a launch gives its tiles to do: its n segments or jobs, each with its
+ * own frames (and, a batch's jobs, channels), which fill whole tiles by
+ * themselves. */
+struct Load {
+    const Seg *s;
+    const GemmArgs *g;
+    uint32_t n;
+    bool batch;                     /* jobs: g[i] with s[i]; else segments: g[0] with every s[i] */
+
+    uint64_t tiles(uint32_t bn, uint32_t bm) const {
+        uint64_t t = 0;
+        for (uint32_t i = 0; i < n; i++)
+            t += (uint64_t)((g[batch ? i : 0].rows + bn - 1) / bn) * ((s[i].T + bm - 1) / bm);
+        return t;
+    }
+    /* tiling i's tiles a CU, the fullest CU's */
+    uint32_t a_cu(int i) const { return (uint32_t)((tiles(kRing[i].bn, kRing[i].bm) + 255) / 256); }
+};
+
 /* The tile for a product in blocks of qb = 32 or 64 inputs, whose time is
  * the blocks' float chains (VALU) and each wave's pass over K more than the
- * loads, so more and smaller tiles pay further than above. Measured (us) on
- * the layer's shapes from 20 to 7500 frames, every tiling:
- *   two 32 x 32 tiles a CU at most: those (blocks of 32, 4096 -> 1024 at 384
- *   frames 13.8 against 18.8 with 64 x 64, at 500 14.6 against 18.8, at 750,
- *   three a CU, 22 against 19.4; 1024 -> 1024 at 137 4.8 against 7.0);
- *   up to a 64 x 64 tile a CU: eight waves (1024 -> 2048 at 500, 256 tiles,
- *   7.8 against 8.8 with four waves);
- *   below two 64 x 64 tiles a CU: in blocks of 32 64 x 32 (1024 -> 4096 at
- *   384 10.4 against 11.4), in blocks of 64, whose chains are half as long,
- *   64 x 64 with three slots (8.8 against 9.4 with 64 x 32), four where the
- *   inputs are deep (4096 -> 1024 at 1200 19.9 against 21.6);
- *   more: 64 x 64 with three slots, or 128 x 128 where whole rounds of one a
- *   CU are at least nine tenths full (1024 -> 4096 in blocks of 64 at 3000
- *   frames, 768 tiles, 30.6 against 34.8; at 2200, 576, 28.6 against 27.7, in
- *   blocks of 32 44.6 against 34.9). */
-static int pick_blocked(uint32_t rows, uint64_t frames, uint32_t ku, uint32_t qb) {
+ * loads, so more and smaller tiles pay further than above. Launches of the
+ * layer's shapes from 17 to 7500 frames, of 2 to 64 segments of 20 to 700
+ * frames and of the layer's q, k, v and positions were measured under every
+ * tiling, and what is best follows the tiles a CU (us):
+ *   two 32 x 32 at most: those (blocks of 32, 4096 -> 1024 at 384 frames 14.5
+ *   against 19.7 with 64 x 64; at 640, three a CU, 24.5 against 20.3);
+ *   one 64 x 64: eight waves (blocks of 32, 1024 -> 2048 at 500 frames 8.5
+ *   against 9.5 with four);
+ *   64 x 32 where they are at most half as many again (blocks of 32: 1024 ->
+ *   4096 at 384 frames, three against two, 10.9 against 11.6 with 64 x 64) or
+ *   fewer (blocks of 64), as short segments have them (blocks of 32, 64 of 20
+ *   frames, 1024 -> 1024, four against four 16.7 against 24.0);
+ *   two 64 x 64: in blocks of 32 four slots (1024 -> 1024 at 1800 frames
+ *   11.7 against 13.0 with 64 x 32, four a CU) or, deep packed inputs, eight
+ *   waves (4096 -> 1024 30.6 against 31.8 and 36.4; row-major, 16 segments of
+ *   128 frames, 40.5 against 38.2); in blocks of 64, whose chains are half as
+ *   long, three slots (1024 -> 4096 at 384 9.2 against 9.5 with
+ *   64 x 32), deep inputs four (4096 -> 1024 at 1200 21.0 against 22.5);
+ *   more: three slots, or 128 x 128 tiles, one of which takes as long as 4 of
+ *   those in blocks of 32 (1024 -> 1024 at 3600 frames, 1 against 4, 18.4
+ *   against 19.7; 1024 -> 4096 at 2500, 3 against 10, 45.0 against 38.5), as
+ *   3.25 in blocks of 64 (1024 -> 4096 at 4210, 5 against 17, 44.4 against
+ *   46.7; at 2200, 3 against 9, 28.8 against 27.0) and as 2.7 from row-major
+ *   activations, which 64 x 64 tiles load less well (16 segments of 200
+ *   frames, 4 against 16, 44.2 against 56.3); three 64 x 64 run together on
+ *   a CU and stay.
+ * silu: the tiles with the fused SiLU quantize only. */
+static int pick_blocked(const Load &l, uint32_t ku, uint32_t qb, bool silu = false) {
     if (g_forced_ring >= 0 && fits(g_forced_ring, ku))
         return g_forced_ring;
-    auto tiles = [&](int i) { return (uint64_t)((rows + kRing[i].bn - 1) / kRing[i].bn) * ((frames + kRing[i].bm - 1) / kRing[i].bm); };
     static const int w8 = ring_index("pipe<64x64w8,2,4>"), s3 = ring_index("pipe<64x64,2,3>"),
                      s4 = ring_index("pipe<64x64,2,4>"), small = ring_index("pipe<32x32,4,4>"),
                      half = ring_index("pipe<64x32,2,3>"), big = ring_index("pipe<128x128w8,1,4>");
-    const uint64_t t128 = tiles(big), t64 = tiles(s3);
+    const uint32_t n64 = l.a_cu(s3), nh = l.a_cu(half), n128 = l.a_cu(big);
+    const bool packed = l.s[0].qstride != 0;
+    const uint32_t worth = qb == 32 ? 48 : packed ? 39 : 32;       /* twelfths */
     int c = s3;
-    if (tiles(small) <= 512 && fits(small, ku))
-        c = small;
-    else if (t64 <= 256)
-        c = w8;
-    else if (t64 < 512)
-        c = qb == 32 ? half : ku >= 32 ? s4 : s3;
-    else if (10 * t128 >= 9 * ((t128 + 255) / 256 * 256))
+    if (!silu && n64 > 3 && worth * n128 <= 12 * n64)
         c = big;
-    return fits(c, ku) ? c : fits(s4, ku) ? s4 : 4;     /* 4 takes any ku: one unit a stage, four slots */
+    else if (l.a_cu(small) <= 2 && fits(small, ku))
+        c = silu ? half : small;
+    else if (n64 == 1)
+        c = w8;
+    else if (qb == 32 ? 2 * nh <= 3 * n64 : 2 * nh < 3 * n64)
+        c = half;
+    else if (n64 == 2)
+        c = qb == 32 ? (ku >= 32 && packed ? w8 : s4) : ku >= 32 ? s4 : s3;
+    return fits(c, ku) ? c : 4;     /* takes any ku: one unit a stage, four slots */
 }
 
 /* whether streamed tiling i (an index of kStream) takes ku units a panel: a
@@ -2145,6 +2179,7 @@ int launch_gemm(const GemmArgs &ga, const SegTable &tab, hipStream_t s, const ch
     g.plain = frames * ga.rows * 4 > kPlainStoreBytes;
     if (frames == 0 || g.rows == 0)
         return 0;
+    const Load load{ tab.s, &g, tab.nseg, false };
     const int mode = g.qb == g.n ? 0 : g.qb % 64 == 0 ? 1 : 2;
     static const char *const modes[] = { "per-column", "blocks of 64k", "blocks of 32k" };
     static thread_local char buf[96];
@@ -2226,13 +2261,12 @@ int launch_gemm(const GemmArgs &ga, const SegTable &tab, hipStream_t s, const ch
     /* blocks of 64 or 32 inputs (the encoder's modes): the pipelined tile
      * the heuristic picks for these frames, if it has a blocked variant */
     if ((mode == 1 && g.qb == 64) || (mode == 2 && g.qb == 32)) {
-        int c = pick_blocked(g.rows, frames, g.ku, g.qb);
+        int c = pick_blocked(load, g.ku, g.qb, g.oqp != nullptr);
         if (!(mode == 1 ? kRing[c].run64 : kRing[c].run32))
             c = fits(6, g.ku) ? 6 : 4;      /* a forced tiling without blocks */
         if (g.oqp && !kRing[c].silu) {
-            /* the fused epilogue is the tiles' of two channel waves of 32 */
-            static const int half = ring_index("pipe<64x32,2,3>");
-            c = kRing[c].bn < 64 && fits(half, g.ku) ? half : 6;
+            /* a forced tiling without the epilogue, or inputs too short */
+            c = 6;
             if (!fits(c, g.ku))
                 return -3;
         }
@@ -2287,7 +2321,7 @@ int launch_gemm_batch(const JobTable &jobs_in, hipStream_t s, const char **name)
             return hipPeekAtLastError() == hipSuccess ? 0 : -1;
         }
     }
-    const int c = mode == 0 ? pick_ring(rows, frames, g0.ku) : pick_blocked(rows, frames, g0.ku, g0.qb);
+    const int c = mode == 0 ? pick_ring(rows, frames, g0.ku) : pick_blocked({ jobs.s, jobs.g, jobs.njobs, true }, g0.ku, g0.qb);
     auto batch = mode == 0 ? kRing[c].batch : mode == 1 ? kRing[c].batch64 : mode == 2 ? kRing[c].batch32 : nullptr;
     if (batch) {
         batch(jobs, s);

@@ -603,6 +603,63 @@ def test_streamed_tiles_walk_every_tile(hip, torch, M, K, N, add, pad):
         assert np.array_equal(bits(o), bits(ref)), (names[key[0]], key[1])
 
 
+# (kind, K, N, qb, each segment's frames) and the tiling it takes: sizes where the tiles of the frames' sum, or a
+# bound on them that another shape was measured for, took one up to half as slow again
+PICKS = [("packed", 1024, 1024, 32, [1800], "pipe<64x64,2,4>"), ("packed", 4096, 1024, 32, [1800], "pipe<64x64w8,2,4>"),
+         ("packed", 1024, 4096, 64, [1700], "pipe<128x128w8,1,4>"),
+         ("rows", 1024, 1024, 32, [417, 171, 413, 100, 369, 123, 396, 256, 297, 234, 406, 121, 311], "pipe<64x64,2,3>"),
+         ("rows", 1024, 4096, 64, [70] * 16, "pipe<128x128w8,1,4>"), ("rows", 1024, 2048, 32, [40] * 16, "pipe<64x64,2,4>"),
+         ("rows", 4096, 1024, 32, [128] * 16, "pipe<64x64,2,4>"), ("rows", 1024, 1024, 32, [20] * 64, "pipe<64x32,2,3>"),
+         ("batch", 1024, 1024, 32, [100, 100, 100, 199], "pipe<64x64w8,2,4>"),
+         ("batch", 1024, 1024, 64, [100, 100, 100, 199], "pipe<64x64w8,2,4>")]
+
+
+@pytest.mark.parametrize("kind,K,N,qb,lens,want", PICKS)
+def test_tilings_follow_the_tiles_a_cu(hip, torch, kind, K, N, qb, lens, want):
+    """One product, a grouped launch and a batch take the tiling that their
+    tiles a CU ask for, counted segment by segment, and its bits are those of
+    the 64 x 64 tile forced."""
+    qbv = qb or K
+    dev = torch.device("cuda")
+    torch.manual_seed(K + N + qb + len(lens))
+    g = synth.rng(K + N)
+    names = [hip.tiling_name(i) for i in range(hip.tilings())]
+    with hip.Q8Matrix(synth.pack_q8(synth.weights(g, N, K)), synth.scales(g, N)) as m:
+        segs = []
+        for t in lens:
+            x = torch.randn(t, K, device=dev)
+            q = torch.zeros((t * K if kind == "rows" else hip.packed_bytes(K, t),), dtype=torch.int8, device=dev)
+            d = torch.empty((t * (K // qbv),), dtype=torch.float32, device=dev)
+            if kind == "rows":
+                hip.quantize_dev(q, d, x, K, qbv, t, K)
+            else:
+                hip.quantize_packed_dev(None, q, d, x, K, t, K, qb=qbv)
+            segs.append((t, q, d))
+
+        def run():
+            outs = [torch.full((t, N), 7.0, dtype=torch.float32, device=dev) for t, _, _ in segs]
+            if kind == "rows":
+                hip.gemm_q8_grouped_dev(m, 0, N, m.dev_scales, None,
+                                        [(o, N, q, d, K, qbv, t) for o, (t, q, d) in zip(outs, segs)], 0)
+            elif kind == "batch":
+                hip.gemm_q8_batch_dev([(o, N, m, 0, N, m.dev_scales, None, q, d, K, t, 0)
+                                       for o, (t, q, d) in zip(outs, segs)], qb=qbv)
+            else:
+                (t, q, d), = segs
+                hip.gemm_q8_packed_dev(outs[0], N, m, 0, N, m.dev_scales, None, q, d, K, t, 0, qb=qbv)
+            torch.cuda.synchronize()
+            return outs, hip.last_kernel().split(" ")[0]
+        say("tiling", kind, K, N, qb, lens)
+        got, name = run()
+        hip.force_tiling(names.index("pipe<64x64,2,4>"))
+        try:
+            ref, forced = run()
+        finally:
+            hip.force_tiling(-1)
+    assert name == want and forced == "pipe<64x64,2,4>"
+    assert all(torch.equal(a.view(torch.int32), b.view(torch.int32)) for a, b in zip(got, ref))
+
+
 def test_default_stream_is_torchs_current_one(hip, torch):
     """Calls without a stream go to torch's current stream: the default one,
     the one of a stream context, another thread's own, and back."""
