@@ -1976,49 +1976,6 @@ static int ring_index(const char *name) {
     return -1;
 }
 
-/* The tile for a product of `frames` frames into `rows` channels. */
-static int pick_ring(uint32_t rows, uint64_t frames, uint32_t ku) {
-    if (g_forced_ring >= 0 && fits(g_forced_ring, ku))
-        return g_forced_ring;
-    auto tiles = [&](int i) { return (uint64_t)((rows + kRing[i].bn - 1) / kRing[i].bn) * ((frames + kRing[i].bm - 1) / kRing[i].bm); };
-    static const int w8 = ring_index("pipe<64x64w8,2,4>"), s3 = ring_index("pipe<64x64,2,3>"),
-                     small = ring_index("pipe<32x32,4,4>");
-    /* measured on the layer's shapes from 20 to 7500 frames (every tiling,
-     * every product): 128 x 128 tiles for five eighths of the CUs or more
-     * take the eight-wave pipelined tile (160 tiles: 4096 -> 1024 at 2500
-     * frames 20.1 us against 21.6 with 64 x 64, 1024 -> 1024 9.0 against 9.0;
-     * 232: at 3600 21.9 against 29.4, 9.8 against 11.8; 1024 -> 2048 at
-     * 1600, 208 tiles, 9.6 against 11.6); where two 32 x 32 tiles a CU hold the whole product,
-     * those (us, 32 x 32 against the best 64 x 64: 1024 -> 1024 at 100 frames
-     * 3.2 against 4.1, at 384 4.1 against 4.3, at 750, where they are three a
-     * CU, 5.1 against 4.8; 4096 -> 1024 at 100 frames 6.0 against 8.5, at 384
-     * 8.0 against 8.8; 1024 -> 640 at 750 4.0 against 4.5); more take 64 x 64
-     * pipelined tiles of two-unit stages: split into two K groups where the
-     * inputs are deep; eight waves of 32 x 16 (two a SIMD) below two tiles a
-     * CU (1024 -> 4096 at 384 frames 6.5 against 7.0 us with four waves);
-     * three slots (three workgroups a CU) from there on; inputs too short for
-     * their slots take the ring, 64 x 64, with longer stages the fewer the
-     * tiles */
-    if (tiles(0) >= 160 && fits(5, ku))
-        return 5;
-    if (tiles(small) <= 512 && fits(small, ku))
-        return small;
-    if (ku >= 32 && tiles(6) < 512 && fits(13, ku))
-        return 13;          /* deep inputs, few tiles: two K groups a tile */
-    const uint64_t t64 = tiles(1);
-    if (t64 < 512 && fits(w8, ku))
-        return w8;
-    if (t64 >= 512 && fits(s3, ku))
-        return s3;
-    if (fits(6, ku))
-        return 6;
-    if (t64 >= 512)
-        return 1;
-    if (t64 >= 256 && ku % 8 == 0)
-        return 2;
-    return ku % 16 == 0 ? 3 : ku % 8 == 0 ? 2 : 1;
-}
-
 /* What a launch gives its tiles to do: its n segments or jobs, each with its
  * own frames (and, a batch's jobs, channels), which fill whole tiles by
  * themselves. */
@@ -2037,6 +1994,56 @@ struct Load {
     /* tiling i's tiles a CU, the fullest CU's */
     uint32_t a_cu(int i) const { return (uint32_t)((tiles(kRing[i].bn, kRing[i].bm) + 255) / 256); }
 };
+
+/* The tile for a whole-row product. What is best of every tiling, measured on
+ * the launches named at pick_blocked, follows the tiles a CU (us):
+ *   128 x 128 on eight waves, one of which takes as long as 2.5 64 x 64 tiles
+ *   (row-major, 4096 -> 1024 at 2500 frames, 1 against 3, 24.3 against 31.6,
+ *   1024 -> 2048 at 2500, 2 against 5, 15.9 against 17.6; packed, 1024 ->
+ *   4096 at 1300, 2 against 6, 13.2 against 14.2); one of packed, not deep
+ *   inputs against three, which run together on a CU, only for 160 tiles and
+ *   inputs of 1024 or more (1024 -> 2048 at 1400 frames, 176, 8.9 in each of
+ *   six runs against 8.7 to 13.2; at 1200, 160, 8.8 against 8.5; 640 -> 1040
+ *   at 2500, 180, 7.9 against 7.5);
+ *   two 32 x 32 at most: those (1024 -> 1024 at 384 frames 4.4 against 4.9
+ *   with 64 x 64; at 750, three a CU, 5.9 against 5.1; 4096 -> 1024 at 384
+ *   7.5 against 8.8);
+ *   64 x 32 where they are less than half as many again as 64 x 64, short
+ *   segments (64 of 20 frames, 1024 -> 1024, 13.2 against 17.2);
+ *   one or two 64 x 64: split into two K groups where the inputs are deep,
+ *   else eight waves of 32 x 16 (two a SIMD; 1024 -> 4096 at 384 frames 6.6
+ *   against 7.0 with four), in a batch's jobs, two a CU, four of 32 x 32 (the
+ *   layer's q, k, v and positions at 300 frames 7.5 against 7.8);
+ *   more: three slots (three workgroups a CU), four row-major ones eight
+ *   waves, in two full rounds (16 segments of 40 frames, 1024 -> 4096, 13.1
+ *   against 14.0);
+ *   inputs of four units, too few for the slots of the 64 x 64 tiles: the
+ *   ring. */
+static int pick_ring(const Load &l, uint32_t ku) {
+    if (g_forced_ring >= 0 && fits(g_forced_ring, ku))
+        return g_forced_ring;
+    static const int w8 = ring_index("pipe<64x64w8,2,4>"), s3 = ring_index("pipe<64x64,2,3>"),
+                     s4 = ring_index("pipe<64x64,2,4>"), k2 = ring_index("pipe<64x64,1,4,k2>"),
+                     small = ring_index("pipe<32x32,4,4>"), half = ring_index("pipe<64x32,2,3>"),
+                     big = ring_index("pipe<128x128w8,1,4>"), ring = ring_index("ring<64x64,1>");
+    const uint32_t n64 = l.a_cu(s3), n128 = l.a_cu(big);
+    const bool rows = l.s[0].qstride == 0, deep = ku >= 32;
+    if (fits(big, ku) && 5 * n128 <= 2 * n64 &&
+        (rows || deep || n64 > 3 || (ku >= 16 && l.tiles(kRing[big].bn, kRing[big].bm) >= 160)))
+        return big;
+    int c = s3;
+    if (l.a_cu(small) <= 2 && fits(small, ku))
+        c = small;
+    else if (n64 > 1 && 2 * l.a_cu(half) < 3 * n64)
+        c = half;
+    else if (n64 <= 2 && deep && fits(k2, ku))
+        c = k2;
+    else if (n64 == 2 && l.batch)
+        c = s4;
+    else if (n64 <= 2 || (n64 == 4 && rows))
+        c = w8;
+    return fits(c, ku) ? c : ring;
+}
 
 /* The tile for a product in blocks of qb = 32 or 64 inputs, whose time is
  * the blocks' float chains (VALU) and each wave's pass over K more than the
@@ -2108,36 +2115,38 @@ static bool stream_spans_fit(const GemmArgs &g, const Seg &sg) {
     return wspan < lim && aspan < lim;
 }
 
-/* The streamed tiling (an index of stream_cfg) for a per-row product of one
- * segment, or -1 for the per-launch tiles: the forced one where it fits;
- * else 256 x 128 streamed tiles where there are at least 400 of them, or,
- * with deep inputs (4096), more than one for two CUs (129: at 4210 frames, 132
- * tiles, 27.2 us against 30.2, at 6000 30.4 against 32.8; at 3600, 116, 27.0
- * against 21.9). Measured at 7500 frames (each product alone): ff
+/* The streamed tiling (an index of stream_cfg) for a per-row product, or -1
+ * for the per-launch tiles: the forced one where it fits; else 256 x 128
+ * streamed tiles where one segment has at least 400 of them, or, with deep
+ * inputs (4096), more than one for two CUs (129: at 4210 frames, 132 tiles,
+ * 27.2 us against 30.2, at 6000 30.4 against 32.8; at 3600, 116, 27.0 against
+ * 21.9; segments, 4096 -> 1024, eight of 520 frames, 160 tiles, 33.2 against
+ * 43.4, eight of 450, 128, 32.9 against 28.3; not those of 2048 inputs or
+ * fewer: 1024 -> 4096, four of 384, 192 tiles, 16.4 against 17.5, but six of
+ * 113, 144, 14.6 against 13.3). Measured at 7500 frames (each product alone): ff
  * up 41-44 against 46-47 us, pw1 24.2 against 25.9, the positions' 14999
  * rows 26-30 against 28-34, ff down 32.7-34.3 against 34.2-36.1; the 236-tile
  * products with 1024 inputs (q, k, v, o, pw2) run faster on the per-launch
  * tiles (two workgroups a CU fill each other's barrier waits where one tile
  * a CU leaves nothing to stream: q 15.3 against 16.5 us, o 18.6 against
- * 19.6). A batch (its rows the largest job's, its frames all jobs') takes
- * 128 x 256 streamed tiles where there are at least 1024 of them: the
+ * 19.6). A batch takes 128 x 256 streamed tiles where there are at least 1024 of them: the
  * attention's q, k, v and positions at 7500 frames 58.2-58.7 us against
  * 64.8-65.7 on the per-launch tiles (61.1-61.4 on 256 x 128) with the batch
  * alone, 63.2 against 64.8 inside the 24-layer sweep (each layer's weights
  * cold). */
-static int pick_stream(uint32_t rows, uint64_t frames, uint32_t ku, bool batch = false) {
+static int pick_stream(const Load &l, uint32_t ku) {
     if (g_forced_ring >= kNRing) {
         const int i = g_forced_ring - kNRing;
         return stream_fits(i, ku) ? i : -1;
     }
-    const int i = batch ? 1 : 0;
+    const int i = l.batch ? 1 : 0;
     if (g_forced_ring >= 0 || !stream_fits(i, ku))
         return -1;
     const StreamCfg &c = *stream_cfg(i);
-    const uint64_t tiles = (uint64_t)((rows + c.bn - 1) / c.bn) * ((frames + c.bm - 1) / c.bm);
-    if (batch)
+    const uint64_t tiles = l.tiles(c.bn, c.bm);
+    if (l.batch)
         return tiles >= 1024 ? i : -1;
-    return tiles >= 400 || (ku >= 64 && tiles > 128) ? i : -1;
+    return (l.n == 1 && tiles >= 400) || (ku >= 64 && tiles > 128) ? i : -1;
 }
 
 template <int WN, int WM, int TN, int TM, int MODE>
@@ -2225,7 +2234,7 @@ int launch_gemm(const GemmArgs &ga, const SegTable &tab, hipStream_t s, const ch
         return hipPeekAtLastError() == hipSuccess ? 0 : -1;
     }
     if (mode == 0 && tab.nseg == 1 && stream_spans_fit(g, tab.s[0])) {
-        const int c = pick_stream(g.rows, frames, g.ku);
+        const int c = pick_stream(load, g.ku);
         if (c >= 0) {
             stream_cfg(c)->run(g, tab, s);
             *name = stream_cfg(c)->name;
@@ -2233,13 +2242,12 @@ int launch_gemm(const GemmArgs &ga, const SegTable &tab, hipStream_t s, const ch
         }
     }
     if (mode == 0 && tab.nseg > 1 && tab.nseg <= (uint32_t)kMaxJobs) {
-        /* the segments as a batch's jobs, one matrix: with deep inputs only
-         * (eight segments, 4210 frames: 4096 -> 1024 28.1 us against 45.6 on
-         * the per-launch tiles, 1024 -> 4096 33.7 against 33.5) */
-        bool rows = g.ku >= 64 || g_forced_ring >= kNRing;
+        /* the segments as a batch's jobs, one matrix; more of them than a
+         * table of jobs holds stay on the per-launch tiles */
+        bool rows = true;
         for (uint32_t i = 0; i < tab.nseg; i++)
             rows = rows && tab.s[i].qstride == 0 && stream_spans_fit(g, tab.s[i]);
-        const int c = rows ? pick_stream(g.rows, frames, g.ku) : -1;
+        const int c = rows ? pick_stream(load, g.ku) : -1;
         if (c >= 0) {
             JobTable t;
             t.njobs = tab.nseg;
@@ -2253,7 +2261,7 @@ int launch_gemm(const GemmArgs &ga, const SegTable &tab, hipStream_t s, const ch
         }
     }
     if (mode == 0) {
-        const int c = pick_ring(g.rows, frames, g.ku);
+        const int c = pick_ring(load, g.ku);
         kRing[c].run(g, tab, s);
         *name = kRing[c].name;
         return hipPeekAtLastError() == hipSuccess ? 0 : -1;
@@ -2294,10 +2302,8 @@ int launch_gemm(const GemmArgs &ga, const SegTable &tab, hipStream_t s, const ch
 }
 
 int launch_gemm_batch(const JobTable &jobs_in, hipStream_t s, const char **name) {
-    uint32_t rows = 0;
     uint64_t frames = 0, outs = 0;
     for (uint32_t j = 0; j < jobs_in.njobs; j++) {
-        rows = jobs_in.g[j].rows > rows ? jobs_in.g[j].rows : rows;
         frames += jobs_in.s[j].T;
         outs += (uint64_t)jobs_in.s[j].T * jobs_in.g[j].rows * 4;
     }
@@ -2306,22 +2312,22 @@ int launch_gemm_batch(const JobTable &jobs_in, hipStream_t s, const char **name)
         jobs.g[j].plain = outs > kPlainStoreBytes;
     if (jobs.njobs == 0 || frames == 0)
         return 0;
-    /* the tiling the jobs would take as one product of their frames; every
-     * job shares the blocks (the caller checks) */
+    /* one tiling for all; every job shares the blocks (the caller checks) */
     const GemmArgs &g0 = jobs.g[0];
+    const Load load{ jobs.s, jobs.g, jobs.njobs, true };
     const int mode = g0.qb == g0.n ? 0 : g0.qb == 64 ? 1 : g0.qb == 32 ? 2 : -1;
     bool spans = true;
     for (uint32_t j = 0; j < jobs.njobs; j++)
         spans = spans && stream_spans_fit(jobs.g[j], jobs.s[j]);
     if (mode == 0 && spans) {
-        const int sc = pick_stream(rows, frames, g0.ku, true);
+        const int sc = pick_stream(load, g0.ku);
         if (sc >= 0) {
             stream_cfg(sc)->batch(jobs, s);
             *name = stream_cfg(sc)->name;
             return hipPeekAtLastError() == hipSuccess ? 0 : -1;
         }
     }
-    const int c = mode == 0 ? pick_ring(rows, frames, g0.ku) : pick_blocked({ jobs.s, jobs.g, jobs.njobs, true }, g0.ku, g0.qb);
+    const int c = mode == 0 ? pick_ring(load, g0.ku) : pick_blocked(load, g0.ku, g0.qb);
     auto batch = mode == 0 ? kRing[c].batch : mode == 1 ? kRing[c].batch64 : mode == 2 ? kRing[c].batch32 : nullptr;
     if (batch) {
         batch(jobs, s);

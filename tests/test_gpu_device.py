@@ -605,7 +605,13 @@ def test_streamed_tiles_walk_every_tile(hip, torch, M, K, N, add, pad):
 
 # (kind, K, N, qb, each segment's frames) and the tiling it takes: sizes where the tiles of the frames' sum, or a
 # bound on them that another shape was measured for, took one up to half as slow again
-PICKS = [("packed", 1024, 1024, 32, [1800], "pipe<64x64,2,4>"), ("packed", 4096, 1024, 32, [1800], "pipe<64x64w8,2,4>"),
+PICKS = [("packed", 1024, 2048, 0, [1400], "pipe<128x128w8,1,4>"), ("packed", 640, 1040, 0, [2500], "pipe<64x64,2,3>"),
+         ("rows", 1024, 4096, 0, [40] * 16, "pipe<64x64w8,2,4>"), ("rows", 1024, 2048, 0, [20] * 64, "pipe<64x32,2,3>"),
+         ("rows", 4096, 1024, 0, [40] * 8, "pipe<32x32,4,4>"), ("rows", 4096, 1024, 0, [450] * 8, "pipe<128x128w8,1,4>"),
+         ("rows", 4096, 1024, 0, [520] * 8, "stream<256x128,2,3,l4>"),
+         ("batch", 1024, 1024, 0, [100, 100, 100, 199], "pipe<64x64w8,2,4>"),
+         ("batch", 1024, 1024, 0, [300, 300, 300, 599], "pipe<64x64,2,4>"),
+         ("packed", 1024, 1024, 32, [1800], "pipe<64x64,2,4>"), ("packed", 4096, 1024, 32, [1800], "pipe<64x64w8,2,4>"),
          ("packed", 1024, 4096, 64, [1700], "pipe<128x128w8,1,4>"),
          ("rows", 1024, 1024, 32, [417, 171, 413, 100, 369, 123, 396, 256, 297, 234, 406, 121, 311], "pipe<64x64,2,3>"),
          ("rows", 1024, 4096, 64, [70] * 16, "pipe<128x128w8,1,4>"), ("rows", 1024, 2048, 32, [40] * 16, "pipe<64x64,2,4>"),
