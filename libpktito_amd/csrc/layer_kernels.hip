@@ -1083,23 +1083,34 @@ static size_t att_fused_lds(uint32_t T, int NW) {
     return ((size_t)NW * 1024 + (size_t)kFQ * att_row(T) + (size_t)kFQ * (128 + 4)) * 4;
 }
 
-/* The waves of the one-kernel attention for T frames and H heads, 0 where
- * the separate kernels are the better ones. Measured (us, 8 heads of 128, one
- * kernel against four): up to a workgroup a CU eight waves (137 frames 15.7
- * against 29.1, 384 25.5 against 46.5; four waves 27.1); then four waves
- * while two workgroups fit a CU's LDS (600 60 against 66, 750 67.5 against
- * 81.8, 820 77 against 85); past that a CU holds one workgroup, and whole
- * rounds of them decide: eight waves where the rounds are full and at most
- * three (1024 109 against 118, 1499 222 against 242, but 1100, its third
- * round nearly empty, 167 against 161, and 2000, a fourth round, 406
- * against 367). */
-static int att_fused_waves(uint32_t T, uint32_t H) {
-    const uint64_t grid = (uint64_t)H * ((T + kFQ - 1) / kFQ), rounds = (grid + 255) / 256;
+/* The waves of the one-kernel attention for T frames and H heads of dk (64 or
+ * 128), 0 where the separate kernels are the better ones. Measured back to
+ * back in a HIP graph (us, one kernel against four; 8 heads of 128 unless
+ * said), 1 to 32 heads of both widths, 17 to 1536 frames:
+ *   up to a workgroup a CU eight waves (137 frames 16.2 against 29.0, 384
+ *   26.4 against 46.0, four waves 27.7; one head of 1499 frames 74 against
+ *   93, of 64 dimensions 59 against 84);
+ *   then four waves while two workgroups fit a CU's LDS (600 60.1 against
+ *   64.8, 750 68.9 against 81.8, 820 77.3 against 86.4), but for long inputs
+ *   only where the rounds of two a CU are at least seven twelfths full (832
+ *   frames: 5 heads, 260 workgroups, 78.3 against 71.9, 10 heads, 520, 122
+ *   against 116, 12 heads, 624, 123 against 131; heads of 64 at 750: 11,
+ *   517, 80.7 against 76.6, 13, 611, 82.2 against 85.1);
+ *   past that a CU holds one workgroup, and whole rounds of them decide:
+ *   eight waves where at most three rounds, of heads of 64 two, are full
+ *   (1024 108 against 117, 1499 223 against 241, 1100, its third round nearly
+ *   empty, 172 against 162; 8 heads of 64: 1000 83 against 92, 1536 176
+ *   against 166; a fourth round loses: 16 heads of 128 at 1000 210 against
+ *   205).
+ * A kernel trace reads both paths longer (384 frames 27.2 against 48.2, 750
+ * 75 against 90, 1499 251 against 279). */
+static int att_fused_waves(uint32_t T, uint32_t H, uint32_t dk) {
+    const uint64_t grid = (uint64_t)H * ((T + kFQ - 1) / kFQ), rounds = (grid + 255) / 256, pairs = (grid + 511) / 512;
     if (grid <= 256)
         return att_fused_lds(T, 8) <= 160 * 1024 && T <= 1536 ? 8 : 0;
     if (2 * att_fused_lds(T, 4) <= 160 * 1024)
-        return 4;
-    return T <= 1536 && rounds <= 3 && 100 * grid >= 95 * 256 * rounds ? 8 : 0;
+        return T <= (dk == 128 ? 768 : 640) || 12 * grid >= 7 * 512 * pairs ? 4 : 0;
+    return T <= 1536 && rounds <= (dk == 128 ? 3 : 2) && 100 * grid >= 95 * 256 * rounds ? 8 : 0;
 }
 
 /* --------------------------------------------------------------- dwq --
@@ -1378,7 +1389,7 @@ int launch_attention(float *of, float *ws, const float *qf, const float *kf, con
     const uint64_t td = (uint64_t)T * D;
     const bool inplace = over(qf, td) || over(kf, td) || over(vf, td) || over(pf, 2 * td - D) || over(bu, D) ||
                          over(bv, D);
-    const int waves = g_att_kind || small || dk > 128 || inplace ? 0 : att_fused_waves(T, H);
+    const int waves = g_att_kind || small || dk > 128 || inplace ? 0 : att_fused_waves(T, H, dk);
     if (waves) {
 #define PK_FUSED(DK, NW) \
     att_fused_kernel<DK, NW><<<H * ((T + kFQ - 1) / kFQ), 64 * NW, att_fused_lds(T, NW), s>>>( \

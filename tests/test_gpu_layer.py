@@ -189,6 +189,33 @@ def test_attention_paths_agree(hip, torch, T, D, H):
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("T,D,H,one", [(832, 640, 5, False), (832, 1280, 10, False), (832, 1536, 12, True), (750, 1280, 10, True),
+                                       (750, 704, 11, False), (600, 704, 11, True), (1499, 512, 8, False),
+                                       (1000, 512, 8, True), (1499, 1024, 8, True), (1100, 1024, 8, False),
+                                       (900, 1024, 16, False), (1536, 128, 1, True), (1537, 128, 1, False)])
+def test_attention_takes_the_one_kernel_where_it_is_faster(hip, torch, T, D, H, one):
+    """Which kernels a length and its heads take, by whether the workspace's
+    scores were written (the one kernel leaves it alone): both sides of each
+    rule, in lengths, in how full the rounds of workgroups are and in the
+    heads' width; both give the same bits."""
+    g = torch.Generator(device="cuda").manual_seed(T + D)
+    q, k, v, p = (torch.randn(n, D, generator=g, device="cuda") for n in (T, T, T, 2 * T - 1))
+    u, b = (0.1 * torch.randn(D, generator=g, device="cuda") for _ in range(2))
+    ws = torch.full((hip.attention_workspace(T, H),), 255, dtype=torch.uint8, device="cuda")
+    outs = []
+    for kind in (0, 2):
+        was = hip.force_attention(kind)
+        try:
+            say("attention", T, D, H, kind)
+            outs.append(torch.full_like(q, 7.0))
+            hip.attention_dev(outs[-1], q, k, v, p, u, b, T, D, H, ws)
+            torch.cuda.synchronize()
+            assert bool((ws == 255).all()) == (one and kind == 0)
+        finally:
+            hip.force_attention(was)
+    assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+
+
 @pytest.mark.parametrize("T,D,H", [(16, 128, 1), (17, 1024, 8), (33, 256, 4), (64, 1024, 8)])
 def test_attention_over_the_values(hip, torch, T, D, H):
     """The output written over the values, which up to 64 frames (one
