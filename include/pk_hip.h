@@ -428,9 +428,10 @@ int pk_hip_force_split(int splits);
 
 /* Tests and tuning: 0 makes every later search load its LSTM, jpred and
  * jout panels from memory each token even where they fit resident (in its
- * workgroups' registers, loaded once a launch:
- * P and J up to 640, at most 2 LSTM layers), 1 restores that; returns the
- * previous setting. Both compute the same tokens. */
+ * workgroups' registers, loaded once a launch: P and J up to 640, at most 2
+ * LSTM layers, at most 2048 rows of jout), 1 restores that; returns the
+ * previous setting. Both compute the same tokens; pk_hip_last_kernel says
+ * which ran, "search_resident" or "search". */
 int pk_hip_force_search_resident(int on);
 
 /* Tests and tuning: forcing the packed quantize's kernel for every later

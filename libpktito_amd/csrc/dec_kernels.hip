@@ -1064,15 +1064,15 @@ size_t search_workspace_bytes(uint32_t L, uint32_t P, uint32_t J, uint32_t rows_
     return up256(512) + up256((size_t)cap * 12) + up256((size_t)L * P * 8) + (loaded > words ? loaded : words) + 256;
 }
 
-int launch_search(SearchArgs &a, void *ws, hipStream_t s) {
+int launch_search(SearchArgs &a, void *ws, hipStream_t s, const char **name) {
     if (a.P == 0 || a.P % 16 || a.P > 1024 || a.J == 0 || a.J % 16 || a.J > 1024 || a.L == 0 ||
         a.L > (uint32_t)kMaxDecLayers || a.rows_out % 16 || a.V + 1 + a.n_dur > a.rows_out || a.n_dur == 0 ||
         a.n_dur > 64 || a.V + 1 > 64 * 32 || 64 * a.kr_p < a.P || a.kr_p > 16 || 64 * a.kr_j < a.J || a.kr_j > 16)
         return -2;
     /* resident: every panel's units and every layer's gate panels fit
-     * (kr <= kResUnits, L <= kResLayers), one workgroup a jpred panel and
-     * two a jout panel's pair (their words are read two a lane of one wave);
-     * else the panels are loaded each token */
+     * (kr <= kResUnits, L <= kResLayers) and at most 64 workgroups have a
+     * jpred panel and two jout panels each at most (the jout panels' words
+     * are read two a lane of one wave); else the panels are loaded each token */
     uint32_t Gr = a.P / 16;
     Gr = Gr > a.J / 16 ? Gr : a.J / 16;
     Gr = Gr > (a.rows_out / 16 + 1) / 2 ? Gr : (a.rows_out / 16 + 1) / 2;
@@ -1116,6 +1116,7 @@ int launch_search(SearchArgs &a, void *ws, hipStream_t s) {
     void *args[] = { &a };
     const void *k = res ? (const void *)search_resident_kernel : (const void *)search_kernel<4, 16>;
     const hipError_t e = hipLaunchCooperativeKernel(k, dim3(G), dim3(res ? 512 : 256), args, 0, s);
+    *name = res ? "search_resident" : "search";
     return e == hipSuccess ? 0 : -1;
 }
 

@@ -1520,8 +1520,9 @@ int pk_hip_search_dev(const pk_hip_decoder *d, const float *f, uint32_t T, int32
     for (uint32_t i = 0; i < d->n_dur; i++)
         a.dur[i] = d->dur[i];
     hipStream_t s = (hipStream_t)stream;
-    PK_LAUNCH(pkq8::launch_search(a, ws, s), "search launch");
-    g_kernel = "search";
+    const char *name = "";
+    PK_LAUNCH(pkq8::launch_search(a, ws, s, &name), "search launch");
+    g_kernel = name;
     /* the flags and the first tokens, which follow them, in one copy */
     constexpr uint32_t kHead = 256;
     struct {

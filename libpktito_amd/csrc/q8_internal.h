@@ -170,11 +170,12 @@ int launch_joint(float *logit, uint32_t *tok_dur, const int8_t *w, uint64_t wstr
 /* The decoder's greedy search in one cooperative launch (dec_kernels.hip):
  * the launch's arguments, the caller filling everything above the
  * workspace's pieces; launch_search carves ws (search_workspace_bytes),
- * zeroes the arrivals, the flag and the state on s, and launches. 0, -2 for
- * shapes it does not take, -1 for a failed call. */
+ * zeroes the arrivals, the flag and the state on s, launches, and names the
+ * kernel that it took. 0, -2 for shapes it does not take, -1 for a failed
+ * call. */
 constexpr int kMaxDecLayers = 8;
 /* the search keeps its panels resident in its workgroups' registers up to
- * this many LSTM layers and units a panel row */
+ * this many LSTM layers and units a panel row (and 128 jout panels) */
 constexpr int kResLayers = 2, kResUnits = 10;
 constexpr int kJointWords = 128 + 64;
 
@@ -203,7 +204,7 @@ struct SearchArgs {
 };
 
 size_t search_workspace_bytes(uint32_t L, uint32_t P, uint32_t J, uint32_t rows_out, uint32_t cap);
-int launch_search(SearchArgs &a, void *ws, hipStream_t s);
+int launch_search(SearchArgs &a, void *ws, hipStream_t s, const char **name);
 /* tests: false makes the search load its panels each token where they
  * would fit resident; returns the previous setting */
 bool set_search_resident(bool on);

@@ -225,7 +225,7 @@ def test_search_in_one_launch(hip, torch, T, seed, scale, resident):
     5 durations): the oracle-driven search's tokens, frames and durations;
     over frames whose scale makes it emit often and others that are mostly
     blank; then the same search again on the same decoder (the state starts
-    from zero each call). Both with the panels resident (registers and LDS,
+    from zero each call). Both with the panels resident (in registers,
     loaded once a launch) and loaded each token."""
     dec = decoder(seed, True)
     V, J, L, P = dec["V"], dec["J"], dec["L"], dec["P"]
@@ -250,6 +250,7 @@ def test_search_in_one_launch(hip, torch, T, seed, scale, resident):
         for call in range(2):
             say("search in one launch", T, seed, call, "resident" if resident else "loaded")
             got = dd.search(fd, T, blank, durs, 10)
+            assert hip.last_kernel() == ("search_resident" if resident else "search")
             assert got == want, (call, len(got), len(want))
     finally:
         hip.force_search_resident(was)
@@ -283,12 +284,14 @@ def test_search_bounded_wait_gives_up(hip, torch):
 
 
 @pytest.mark.parametrize("P,L,J,V,durs", [(1024, 1, 512, 2000, [0, 1, 2]), (256, 3, 768, 100, [0, 1, 2, 4]),
-                                          (320, 2, 320, 500, [0, 1, 2, 3, 4]), (64, 2, 96, 30, [1, 2])])
+                                          (320, 2, 320, 500, [0, 1, 2, 3, 4]), (64, 2, 96, 30, [1, 2]),
+                                          (64, 1, 96, 2047, [0, 1, 2, 3, 4])])
 def test_search_in_one_launch_other_shapes(hip, torch, P, L, J, V, durs):
     """The one-launch search beyond the model's shapes: prediction widths up
     to 1024 (16 units a panel row, where the panels are loaded each token),
     one and three LSTM layers, a joint wider than the prediction, a
-    vocabulary of 2000, durations without 0; its tokens, frames and
+    vocabulary of 2000, one whose 129 panels are one too many to keep,
+    durations without 0; its tokens, frames and
     durations the oracle-driven search's, with the panels resident where
     they fit and loaded each token everywhere."""
     dec = synth.decoder_weights(synth.rng(P + L + J), P=P, L=L, J=J, V=V, n_dur=len(durs))
@@ -315,6 +318,8 @@ def test_search_in_one_launch_other_shapes(hip, torch, P, L, J, V, durs):
                 got = dd.search(fd, T, blank, durs, 10)
             finally:
                 hip.force_search_resident(was)
+            fit = P <= 640 and J <= 640 and L <= 2 and (V + 1 + len(durs) + 15) // 16 <= 128
+            assert hip.last_kernel() == ("search_resident" if resident and fit else "search")
             assert got == want, (resident, len(got), len(want))
     finally:
         dd.release()
@@ -362,6 +367,7 @@ def test_search_resident_edges(hip, torch, P, L, J, V, durs, mark):
         fd = dev(torch, np.concatenate([np.zeros(1, np.float32), frames.reshape(-1)]))
         say("resident search", P, L, J, V, len(durs), mark)
         got = dd.search(None, T, blank, durs, 3, f_ptr=fd.data_ptr() + 4)
+        assert hip.last_kernel() == "search_resident"
     finally:
         dd.release()
     assert got == want and len(want) > 0
