@@ -1987,9 +1987,11 @@ struct Load {
 
     uint64_t tiles(uint32_t bn, uint32_t bm) const {
         uint64_t t = 0;
-        for (uint32_t i = 0; i < n; i++)
-            t += (uint64_t)((g[batch ? i : 0].rows + bn - 1) / bn) * ((s[i].T + bm - 1) / bm);
-        return t;
+        for (uint32_t i = 0; i < n; i++) {
+            const uint32_t m = (s[i].T + bm - 1) / bm;
+            t += batch ? (uint64_t)m * ((g[i].rows + bn - 1) / bn) : m;
+        }
+        return batch ? t : t * ((g[0].rows + bn - 1) / bn);
     }
     /* tiling i's tiles a CU, the fullest CU's */
     uint32_t a_cu(int i) const { return (uint32_t)((tiles(kRing[i].bn, kRing[i].bm) + 255) / 256); }
