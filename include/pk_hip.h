@@ -273,8 +273,10 @@ int pk_hip_layernorm_dev(float *x, uint32_t T, uint32_t n, const float *w, const
  * products' outputs q, k,
  * v [T][D] and the positions' p [2T - 1][D] with the biases u and v [D]:
  * Transformer-XL's scores, the softmax, the weighted values, each output
- * the chain pk_k_gemm_f32 and pk_k_softmax make. The scores live in ws,
- * pk_hip_attention_workspace(T, H) bytes. */
+ * the chain pk_k_gemm_f32 and pk_k_softmax make. ws has
+ * pk_hip_attention_workspace(T, H) bytes, where the scores live if the call
+ * takes the separate kernels (the one kernel keeps them on the chip and
+ * leaves ws alone); which of them a call takes is a matter of its sizes. */
 size_t pk_hip_attention_workspace(uint32_t T, uint32_t H);
 int pk_hip_attention_dev(float *o, const float *q, const float *k, const float *v, const float *p,
                          const float *bias_u, const float *bias_v, uint32_t T, uint32_t D, uint32_t H, void *ws,

@@ -1005,14 +1005,15 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void att_fused_kernel(float *__res
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    /* four groups on their way: 2048 clocks of products */
     v4f pa[4], pb[4];
     auto pload = [&](v4f (&pr)[4], uint32_t j0) {
 #pragma unroll
         for (int k = 0; k < 4; k++)
             pr[k] = *(const v4f *)(e + min(j0, Ts - 20) + 4 * k);
     };
-    /* three groups of values on their way, one of probabilities */
+    /* four groups of values in registers, three of them on their way while
+     * one is multiplied (512 clocks of products a group); the probabilities
+     * one group ahead */
     Keys v0 = vload(0), v1 = vload(16), v2 = vload(32), v3 = vload(48);
     uint32_t j0 = 0;
     pload(pa, 0);
@@ -1102,8 +1103,8 @@ static size_t att_fused_lds(uint32_t T, int NW) {
  *   empty, 172 against 162; 8 heads of 64: 1000 83 against 92, 1536 176
  *   against 166; a fourth round loses: 16 heads of 128 at 1000 210 against
  *   205).
- * A kernel trace reads both paths longer (384 frames 27.2 against 48.2, 750
- * 75 against 90, 1499 251 against 279). */
+ * A kernel trace reads both paths longer (384 frames 27.1 against 47.1, 750
+ * 75 against 89, 1499 249 against 283). */
 static int att_fused_waves(uint32_t T, uint32_t H, uint32_t dk) {
     const uint64_t grid = (uint64_t)H * ((T + kFQ - 1) / kFQ), rounds = (grid + 255) / 256, pairs = (grid + 511) / 512;
     if (grid <= 256)

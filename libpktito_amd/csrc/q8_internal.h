@@ -67,8 +67,8 @@ struct GemmArgs {
     uint32_t qb, nb;            /* block inputs, blocks a column */
     int add;
     int rmode;                  /* 0 nearest, 1 upward, 2 downward, 3 toward zero */
-    /* with oqp set (blocked products on 64 x 64 pipelined tiles, all rows of
-     * the matrix, nearest rounding): the outputs are not stored but SiLU'd and
+    /* with oqp set (blocked products on the pipelined tiles of two channel
+     * waves of 32, all rows of the matrix, nearest rounding): the outputs are not stored but SiLU'd and
      * quantized in blocks of oqb into the packed copy oqp and the scales od,
      * the next product's activations, as a SiLU quantize of them would */
     int8_t *oqp = nullptr;
