@@ -2004,7 +2004,8 @@ struct Load {
  *   1024 -> 2048 at 2500, 2 against 5, 15.9 against 17.6; packed, 1024 ->
  *   4096 at 1300, 2 against 6, 13.2 against 14.2); one of packed, not deep
  *   inputs against three, which run together on a CU, only for 160 tiles and
- *   inputs of 1024 or more (1024 -> 2048 at 1400 frames, 176, 8.9 in each of
+ *   inputs of 1024 or more, or too few for 64 x 64 (256 -> 1024 at 2500
+ *   frames 6.7 against 7.8 with the ring) (1024 -> 2048 at 1400 frames, 176, 8.9 in each of
  *   six runs against 8.7 to 13.2; at 1200, 160, 8.8 against 8.5; 640 -> 1040
  *   at 2500, 180, 7.9 against 7.5);
  *   two 32 x 32 at most: those (1024 -> 1024 at 384 frames 4.4 against 4.9
@@ -2031,7 +2032,8 @@ static int pick_ring(const Load &l, uint32_t ku) {
     const uint32_t n64 = l.a_cu(s3), n128 = l.a_cu(big);
     const bool rows = l.s[0].qstride == 0, deep = ku >= 32;
     if (fits(big, ku) && 5 * n128 <= 2 * n64 &&
-        (rows || deep || n64 > 3 || (ku >= 16 && l.tiles(kRing[big].bn, kRing[big].bm) >= 160)))
+        (rows || deep || n64 > 3 ||
+         ((ku >= 16 || !fits(s3, ku)) && l.tiles(kRing[big].bn, kRing[big].bm) >= 160)))
         return big;
     int c = s3;
     if (l.a_cu(small) <= 2 && fits(small, ku))
@@ -2070,11 +2072,13 @@ static int pick_ring(const Load &l, uint32_t ku) {
  *   more: three slots, or 128 x 128 tiles, one of which takes as long as 4 of
  *   those in blocks of 32 (1024 -> 1024 at 3600 frames, 1 against 4, 18.4
  *   against 19.7; 1024 -> 4096 at 2500, 3 against 10, 45.0 against 38.5), as
- *   3.25 in blocks of 64 (1024 -> 4096 at 4210, 5 against 17, 44.4 against
- *   46.7; at 2200, 3 against 9, 28.8 against 27.0) and as 2.7 from row-major
- *   activations, which 64 x 64 tiles load less well (16 segments of 200
- *   frames, 4 against 16, 44.2 against 56.3); three 64 x 64 run together on
- *   a CU and stay.
+ *   3.67 there from row-major activations of 1536 inputs on (3072 -> 3072 at
+ *   5000, 4 against 15, 154 against 167), as 3.25 in blocks of 64 (1024 ->
+ *   4096 at 4210, 5 against 17, 44.4 against 46.7; at 2200, 3 against 9, 28.8
+ *   against 27.0), 3.5 below 1024 inputs (512 -> 4096 at 2500, 3 against 10,
+ *   21.4 against 20.0), and as 2.7 from row-major activations, which 64 x 64
+ *   tiles load less well (16 segments of 200 frames, 4 against 16, 44.2
+ *   against 56.3); three 64 x 64 run together on a CU and stay.
  * silu: the tiles with the fused SiLU quantize only. */
 static int pick_blocked(const Load &l, uint32_t ku, uint32_t qb, bool silu = false) {
     if (g_forced_ring >= 0 && fits(g_forced_ring, ku))
@@ -2084,7 +2088,7 @@ static int pick_blocked(const Load &l, uint32_t ku, uint32_t qb, bool silu = fal
                      half = ring_index("pipe<64x32,2,3>"), big = ring_index("pipe<128x128w8,1,4>");
     const uint32_t n64 = l.a_cu(s3), nh = l.a_cu(half), n128 = l.a_cu(big);
     const bool packed = l.s[0].qstride != 0;
-    const uint32_t worth = qb == 32 ? 48 : packed ? 39 : 32;       /* twelfths */
+    const uint32_t worth = qb == 32 ? (packed || ku < 24 ? 48 : 44) : !packed ? 32 : ku < 16 ? 42 : 39;  /* twelfths */
     int c = s3;
     if (!silu && n64 > 3 && worth * n128 <= 12 * n64)
         c = big;

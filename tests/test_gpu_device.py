@@ -615,6 +615,9 @@ PICKS = [("packed", 1024, 2048, 0, [1400], "pipe<128x128w8,1,4>"), ("packed", 64
          ("packed", 1024, 4096, 64, [1700], "pipe<128x128w8,1,4>"),
          ("rows", 1024, 1024, 32, [417, 171, 413, 100, 369, 123, 396, 256, 297, 234, 406, 121, 311], "pipe<64x64,2,3>"),
          ("rows", 1024, 4096, 64, [70] * 16, "pipe<128x128w8,1,4>"), ("rows", 1024, 2048, 32, [40] * 16, "pipe<64x64,2,4>"),
+         ("rows", 1024, 1024, 64, [40] * 8, "pipe<32x32,4,4>"), ("rows", 4096, 1024, 32, [16] * 8, "pipe<32x32,4,4>"),
+         ("rows", 4096, 1024, 64, [70] * 8, "pipe<64x64w8,2,4>"), ("rows", 1024, 1024, 64, [185] * 13, "pipe<64x64,2,3>"),
+         ("rows", 2048, 3072, 32, [3600], "pipe<128x128w8,1,4>"), ("rows", 1024, 4096, 32, [2500], "pipe<64x64,2,3>"),
          ("rows", 4096, 1024, 32, [128] * 16, "pipe<64x64,2,4>"), ("rows", 1024, 1024, 32, [20] * 64, "pipe<64x32,2,3>"),
          ("batch", 1024, 1024, 32, [100, 100, 100, 199], "pipe<64x64w8,2,4>"),
          ("batch", 1024, 1024, 64, [100, 100, 100, 199], "pipe<64x64w8,2,4>")]
